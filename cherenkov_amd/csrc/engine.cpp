@@ -2170,7 +2170,7 @@ uint32_t ChkEngine::pf_dense_rows(uint32_t T, uint32_t pos0) const {
 PfFlashLaunch ChkEngine::pf_flash_launch(uint32_t T, uint32_t pos0) {
     const uint64_t key = (uint64_t)T << 32 | pos0;
     if (key != pf.fa_key) {
-        const PfFlashPlan p = pf_flash_plan(T, pos0, std::max<uint32_t>(1, ncu / D.nkv));
+        const PfFlashPlan p = pf_flash_split(T, pos0, (uint32_t)fa_wmax(pf.cap));
         const uint64_t rmax = (pf.cap + 15) / 16, wmax = fa_wmax(pf.cap);
         if (p.seg.size() > rmax * FA_MAXSEG || p.merge.size() > wmax || p.nslots > 2 * wmax)
             throw std::runtime_error("flash attention plan exceeds its buffers");
@@ -3326,11 +3326,12 @@ int chk_fill_u8(void* dst, uint32_t value, uint64_t n, void* stream) {
     })
 }
 
-int chk_pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
-                      uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge) {
+static int flash_plan_out(PfFlashPlan (*make)(uint32_t, uint32_t, uint32_t), uint32_t T, uint32_t pos0, uint32_t max_wg,
+                          uint32_t* W, uint32_t* nslots, uint32_t* seg, uint64_t seg_cap, uint32_t* merge,
+                          uint64_t merge_cap, uint32_t* nmerge) {
     CHK_TRY({
         ensure(T >= 1 && max_wg >= 1, "T and max_wg must be positive");
-        const PfFlashPlan p = pf_flash_plan(T, pos0, max_wg);
+        const PfFlashPlan p = make(T, pos0, max_wg);
         ensure(p.seg.size() * 4 <= seg_cap && p.merge.size() * 4 <= merge_cap, "plan buffers too small");
         *W = p.W;
         *nslots = p.nslots;
@@ -3338,6 +3339,16 @@ int chk_pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, u
         memcpy(seg, p.seg.data(), p.seg.size() * sizeof(uint4));
         if (!p.merge.empty()) memcpy(merge, p.merge.data(), p.merge.size() * sizeof(uint4));
     })
+}
+
+int chk_pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
+                      uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge) {
+    return flash_plan_out(pf_flash_plan, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
+}
+
+int chk_pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
+                       uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge) {
+    return flash_plan_out(pf_flash_split, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
 }
 
 int chk_copy_f32(float* dst, const float* src, uint64_t n, void* stream) {

@@ -465,7 +465,9 @@ bool launch_pf_gemm_args(const PfGemmArgs& a, int epi, uint32_t grid_y, hipStrea
 // for a whole block; row block ~0 ends the list), and per split row block
 // a merge entry (row block, first slot, pieces, 0).
 constexpr uint32_t FA_MAXSEG = 6;
-constexpr int FA_MAXP = 4;  // pieces of a split row block
+constexpr int FA_MAXP = 4;  // pieces of a split row block under pf_flash_plan
+constexpr uint32_t FA_MINSHARE = 3;   // tiles of a workgroup's share under pf_flash_split
+constexpr uint32_t FA_MAXJOIN = 256;  // pieces of a row block k_pf_flash_join takes
 struct PfFlashPlan {
     uint32_t W = 0;            // workgroups per kv head
     uint32_t nslots = 0;       // partial slots per kv head
@@ -473,6 +475,9 @@ struct PfFlashPlan {
     std::vector<uint4> merge;  // [split row blocks]
 };
 PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg);
+// the plan the engine takes: pf_flash_plan, or where the chunk has fewer row
+// blocks than max_wg, its steps over more workgroups than row blocks
+PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg);
 struct PfFlashLaunch {         // a plan uploaded to the device
     const uint4* seg;
     const uint4* merge;

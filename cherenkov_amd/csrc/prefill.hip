@@ -2080,7 +2080,7 @@ namespace chk {
 // to the workgroups in equal shares: row blocks in zigzag order (first,
 // last, second, ...), the sequence cut into W equal ranges, so a workgroup
 // runs a few segments (row block, tile range); a row block cut between
-// workgroups leaves unnormalised partials (m, l, o) that k_pf_flash_merge
+// workgroups leaves unnormalised partials (m, l, o) that k_pf_flash_join
 // joins.  Within a segment, wave w serves the kv head's query head w
 // (GQA: the group's waves share every staged K/V tile).  Per
 // 32-token tile the workgroup dequantises K and V (int8 x fp16 scale,
@@ -2338,62 +2338,49 @@ __global__ void __launch_bounds__(64 * G) k_pf_flash(PfFlashArgs a) {
 // Joins the pieces of the row blocks a flash plan split: per row, head and
 // dim, o = sum_k o_k e^(m_k - M) / sum_k l_k e^(m_k - M) with M = max_k m_k
 // (a piece whose tokens a row cannot see holds m = -inf, l = 0), times the
-// sigmoid gate.  Workgroup (entry, row) of kv head blockIdx.z; thread d
-// takes dims d, d + 256 of every head, all loads issued before the sums.
-template <int G, int HD>
-__global__ void __launch_bounds__(256) k_pf_flash_merge(PfFlashArgs a, const uint4* __restrict__ merge) {
-    constexpr int DPT = (HD + CHK_WG - 1) / CHK_WG;
+// sigmoid gate.  Workgroup (entry, row, query head); the pieces' weights
+// e^(m_k - M) / L meet in LDS (np <= FA_MAXJOIN), then thread d sums dim d
+// over the pieces, eight loads in flight.
+__global__ void __launch_bounds__(256) k_pf_flash_join(PfFlashArgs a, const uint4* __restrict__ merge, uint32_t G,
+                                                       uint32_t hd) {
+    __shared__ float sm[FA_MAXJOIN], red[8];
     const uint4 me = merge[blockIdx.x];  // (row block, first slot, pieces, 0)
-    const uint32_t row = blockIdx.y, hk = blockIdx.z, r = me.x * FA_ROWS + row, np = me.z;
+    const uint32_t row = blockIdx.y, hk = blockIdx.z / G, g = blockIdx.z % G, t = threadIdx.x;
+    const uint32_t r = me.x * FA_ROWS + row, np = me.z;
     if (r >= a.T) return;
-    const float* __restrict__ part = a.part;
-    const float* __restrict__ qraw = a.q_raw;
-    float* __restrict__ outp = a.out;
-    const size_t ps = (size_t)FA_ROWS * G * (2 + HD);  // floats per slot
-    const float* p0 = part + ((size_t)hk * a.nslots + me.y) * ps + (size_t)row * G * (2 + HD);
-    float mk[G][FA_MAXP], lk[G][FA_MAXP], ok[G][FA_MAXP][DPT], gate[G][DPT];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const float* q = p0 + (size_t)g * (2 + HD);
-#pragma unroll
-        for (int k = 0; k < FA_MAXP; ++k) {
-            const bool on = (uint32_t)k < np;
-            mk[g][k] = on ? q[k * ps] : -INFINITY;
-            lk[g][k] = on ? q[k * ps + 1] : 0.0f;
-#pragma unroll
-            for (int j = 0; j < DPT; ++j) {
-                const uint32_t d = threadIdx.x + j * CHK_WG;
-                ok[g][k][j] = on && d < (uint32_t)HD ? q[k * ps + 2 + d] : 0.0f;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < DPT; ++j) {
-            const uint32_t d = min(threadIdx.x + j * CHK_WG, (uint32_t)HD - 1);
-            gate[g][j] = qraw[((size_t)r * a.nh + hk * G + g) * 2 * HD + HD + d];
-        }
+    const size_t ps = (size_t)FA_ROWS * G * (2 + hd);  // floats per slot
+    const float* __restrict__ p0 = a.part + ((size_t)hk * a.nslots + me.y) * ps + ((size_t)row * G + g) * (2 + hd);
+    const uint32_t h = hk * G + g, dc = min(t, hd - 1);
+    const float gate = a.q_raw[((size_t)r * a.nh + h) * 2 * hd + hd + dc];
+    float m = -INFINITY, l = 0.0f;
+    if (t < np) {
+        m = p0[t * ps];
+        l = p0[t * ps + 1];
     }
+    const float M = block_max(m, red);
+    const float e = m == -INFINITY ? 0.0f : expf(m - M);
+    const float L = block_sum(l * e, red);
+    if (t < np) sm[t] = e;
+    __syncthreads();
+    const float* __restrict__ po = p0 + 2 + dc;
+    float O = 0.0f;
+    uint32_t k = 0;
+    for (; k + 8 <= np; k += 8) {
+        float v[8];
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        float M = -INFINITY;
+        for (int j = 0; j < 8; ++j) v[j] = po[(k + j) * ps];
 #pragma unroll
-        for (int k = 0; k < FA_MAXP; ++k) M = fmaxf(M, mk[g][k]);
-        float e[FA_MAXP], L = 0.0f;
-#pragma unroll
-        for (int k = 0; k < FA_MAXP; ++k) {
-            e[k] = mk[g][k] == -INFINITY ? 0.0f : expf(mk[g][k] - M);
-            L += lk[g][k] * e[k];
-        }
-        const float inv = 1.0f / L;
-#pragma unroll
-        for (int j = 0; j < DPT; ++j) {
-            const uint32_t d = threadIdx.x + j * CHK_WG;
-            if (d >= (uint32_t)HD) continue;
-            float O = 0.0f;
-#pragma unroll
-            for (int k = 0; k < FA_MAXP; ++k) O += ok[g][k][j] * e[k];
-            outp[(size_t)r * a.nh * HD + (size_t)(hk * G + g) * HD + d] = O * inv * sigmoidf_(gate[g][j]);
-        }
+        for (int j = 0; j < 8; ++j) O += v[j] * sm[k + j];
     }
+    {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = po[min(k + j, np - 1) * ps];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (k + j < np) O += v[j] * sm[k + j];
+    }
+    if (t < hd) a.out[(size_t)r * a.nh * hd + (size_t)h * hd + t] = O * (1.0f / L) * sigmoidf_(gate);
 }
 
 // Deals every kv head's (row block, tile) steps to max_wg workgroups in
@@ -2458,6 +2445,46 @@ PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg) {
     return p;
 }
 
+// The plan of a chunk with fewer row blocks than workgroups (a short prompt
+// or message, mostly behind a long context): every kv head's steps, row
+// block after row block, cut into equal ranges over up to max_wg
+// workgroups of at least FA_MINSHARE tiles each, so a row block is split
+// over as many workgroups as its context fills.  One workgroup per row
+// block (pf_flash_plan's least) left 70 rows behind 5001 tokens on 10
+// workgroups: 673 us a layer, against 48 split + 8 to join; 333 behind 1500:
+// 264 -> 67 + 12.
+// A range costs its queries and its partial once, about two tiles' time.
+PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg) {
+    const uint32_t R = (T + FA_ROWS - 1) / FA_ROWS;
+    std::vector<uint64_t> first(R + 1, 0);
+    for (uint32_t rb = 0; rb < R; ++rb)
+        first[rb + 1] = first[rb] + (pos0 + std::min(rb * FA_ROWS + FA_ROWS - 1, T - 1)) / FA_TOK + 1;
+    const uint64_t total = first[R];
+    const uint32_t W = (uint32_t)std::min<uint64_t>({max_wg, total / FA_MINSHARE, (uint64_t)FA_MAXJOIN - 1});
+    if (R >= max_wg || W <= R) return pf_flash_plan(T, pos0, max_wg);
+    PfFlashPlan p;
+    p.W = W;
+    p.seg.assign((size_t)W * FA_MAXSEG, make_uint4(~0u, 0, 0, 0));
+    std::vector<uint32_t> nseg(W, 0);
+    for (uint32_t rb = 0; rb < R; ++rb) {
+        const uint32_t slot0 = p.nslots;
+        // the ranges [k total / W, (k + 1) total / W) that meet this row block
+        uint32_t k = (uint32_t)(first[rb] * W / total);
+        while (k > 0 && k * total / W > first[rb]) --k;
+        while (k + 1 < W && (k + 1) * total / W <= first[rb]) ++k;
+        const bool split = (k + 1) * total / W < first[rb + 1];
+        for (; k < W && k * total / W < first[rb + 1]; ++k) {
+            const uint64_t lo = std::max(first[rb], k * total / W), hi = std::min(first[rb + 1], (k + 1) * total / W);
+            if (lo >= hi) continue;
+            if (nseg[k] == FA_MAXSEG) return pf_flash_plan(T, pos0, max_wg);
+            p.seg[(size_t)k * FA_MAXSEG + nseg[k]++] =
+                make_uint4(rb, (uint32_t)(lo - first[rb]), (uint32_t)(hi - first[rb]), split ? p.nslots++ : ~0u);
+        }
+        if (split) p.merge.push_back(make_uint4(rb, slot0, p.nslots - slot0, 0));
+    }
+    return p;
+}
+
 void launch_pf_flash(const float* q_ready, const float* q_raw, const KvDev& kv, float* out, uint32_t T, uint32_t pos0,
                      uint32_t nh, uint32_t nkv, uint32_t hd, float scale, const PfFlashLaunch& plan, hipStream_t st) {
     if (nkv == 0 || nh % nkv || nh / nkv > 8 || (hd != 128 && hd != 256))
@@ -2467,20 +2494,13 @@ void launch_pf_flash(const float* q_ready, const float* q_raw, const KvDev& kv, 
         throw std::runtime_error("flash prefill needs its plan");
     PfFlashArgs a{q_ready, q_raw, kv, out, T, pos0, nh, nkv, scale, plan.seg, plan.part, plan.nslots};
     const dim3 grid(plan.W, nkv);
-    const dim3 mgrid(plan.nmerge, FA_ROWS, nkv);
 #define CHK_FA(HDV)                                                                                      \
     switch (nh / nkv) {                                                                                  \
     case 1: k_pf_flash<HDV, 1><<<grid, 64, 0, st>>>(a); break;                                           \
     case 2: k_pf_flash<HDV, 2><<<grid, 128, 0, st>>>(a); break;                                          \
     case 3: case 4: k_pf_flash<HDV, 4><<<grid, 256, 0, st>>>(a); break;                                  \
     default: k_pf_flash<HDV, 8><<<grid, 512, 0, st>>>(a); break;                                         \
-    }                                                                                                    \
-    if (plan.nmerge) switch (nh / nkv) {                                                                 \
-        case 1: k_pf_flash_merge<1, HDV><<<mgrid, CHK_WG, 0, st>>>(a, plan.merge); break;                \
-        case 2: k_pf_flash_merge<2, HDV><<<mgrid, CHK_WG, 0, st>>>(a, plan.merge); break;                \
-        case 3: case 4: k_pf_flash_merge<4, HDV><<<mgrid, CHK_WG, 0, st>>>(a, plan.merge); break;        \
-        default: k_pf_flash_merge<8, HDV><<<mgrid, CHK_WG, 0, st>>>(a, plan.merge); break;               \
-        }
+    }
     if (nh / nkv != 1 && nh / nkv != 2 && nh / nkv != 4 && nh / nkv != 8)
         throw std::runtime_error("flash prefill takes 1, 2, 4 or 8 query heads per kv head");
     if (hd == 256) {
@@ -2489,6 +2509,8 @@ void launch_pf_flash(const float* q_ready, const float* q_raw, const KvDev& kv, 
         CHK_FA(128)
     }
 #undef CHK_FA
+    if (plan.nmerge)
+        k_pf_flash_join<<<dim3(plan.nmerge, FA_ROWS, nh), CHK_WG, 0, st>>>(a, plan.merge, nh / nkv, hd);
 }
 
 }  // namespace chk

@@ -219,6 +219,12 @@ int chk_time_blocks(ChkEngine* e, int kind, uint32_t nb, const uint32_t* layers,
  * partial slots. */
 int chk_pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
                       uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge);
+/* The plan the engine launches, in the same form: chk_pf_flash_plan's, or
+ * where the chunk has fewer 16-row blocks than max_wg, its steps cut over
+ * up to max_wg workgroups, a row block over any number of them (W <=
+ * max_wg, slots < W + row blocks). */
+int chk_pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
+                       uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge);
 
 /* Time the decode step on the engine's stream: runs `steps` step_rows(1)
  * + commit pairs, returns milliseconds per step (HIP events). */
