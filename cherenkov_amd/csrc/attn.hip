@@ -324,6 +324,69 @@ __global__ void __launch_bounds__(256) k_qsa_score(AttnArgs a) {
     }
 }
 
+// Block scores of prefill rows (block keys cached): the same dots as f32
+// matrix products.  Workgroup: 16 rows, whose index queries sit in LDS, by
+// QP_BLK blocks; a wave takes 16-block tiles, every fourth, and sums each
+// head's relu on v_mfma_f32_16x16x4_f32 (A lane l: row l % 16, B lane l:
+// block l % 16, both holding dims (l / 16) ihd / 4 .. + ihd / 4 of the
+// contraction, whose order is free as long as both agree; D lane l: block
+// l % 16, rows 4 (l / 16) .. + 4).  The next tile's keys are requested
+// before the current one's products.  On wave dots (k_qsa_score, a row a
+// workgroup column) the 2950 rows past the budget of a 5000-token prompt
+// (4 heads of 128) took 47 launches of 28 us; this way 2 of 34.
+constexpr uint32_t QP_BLK = 256;
+typedef float f4v __attribute__((ext_vector_type(4)));
+
+template <int DPL>
+__global__ void __launch_bounds__(256) k_pf_qsa_score(AttnArgs a, uint32_t nr) {
+    constexpr uint32_t D = 64 * DPL, DK = D / 4, DP = DK + 4;  // a quarter's dims, padded in LDS
+    extern __shared__ __align__(16) float sq[];                // [inh][4 quarters][16 rows][DP]
+    const uint32_t r0 = blockIdx.y * 16, t = threadIdx.x, lane = t & 63, w = wave_id();
+    const uint32_t col = lane & 15, kq = lane >> 4;
+    const uint32_t nblk = (a.pos[min(r0 + 15, nr - 1)] + 1) / a.ratio;  // of the tile's last row
+    const uint32_t b0 = blockIdx.x * QP_BLK, b1 = min(b0 + QP_BLK, nblk);
+    if (b0 >= nblk) return;
+    for (uint32_t i = t; i < 16 * a.inh * D; i += CHK_WG) {
+        const uint32_t r = i / (a.inh * D), hd = i % (a.inh * D), h = hd / D, d = hd % D;
+        sq[((h * 4 + d / DK) * 16 + r) * DP + d % DK] = a.iq_ready[(size_t)min(r0 + r, nr - 1) * a.inh * D + hd];
+    }
+    const float* keys = a.kv[0].block_k + (size_t)kq * DK;
+    float4 kn[DK / 4];
+    auto fetch = [&](uint32_t blk) __attribute__((always_inline)) {
+        const float4* kp = reinterpret_cast<const float4*>(keys + (size_t)min(blk + col, nblk - 1) * D);
+#pragma unroll
+        for (uint32_t j = 0; j < DK / 4; ++j) kn[j] = kp[j];
+    };
+    fetch(b0 + w * 16);
+    __syncthreads();
+    const float rs = sqrtf((float)D);
+    for (uint32_t blk = b0 + w * 16; blk < b1; blk += 64) {
+        float4 k[DK / 4];
+#pragma unroll
+        for (uint32_t j = 0; j < DK / 4; ++j) k[j] = kn[j];
+        fetch(blk + 64);
+        f4v s = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (uint32_t h = 0; h < a.inh; ++h) {
+            const float4* qp = reinterpret_cast<const float4*>(&sq[((h * 4 + kq) * 16 + col) * DP]);
+            f4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (uint32_t j = 0; j < DK / 4; ++j) {
+                const float4 q = qp[j];
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q.x, k[j].x, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q.y, k[j].y, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q.z, k[j].z, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q.w, k[j].w, acc, 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] += fmaxf(acc[i], 0.0f);
+        }
+        if (blk + col < nblk)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (r0 + kq * 4 + i < nr) a.bscore[(size_t)(r0 + kq * 4 + i) * a.max_blocks + blk + col] = s[i] / rs;
+    }
+}
+
 // The top kblk of a row's nblk block scores by (score desc, block asc):
 // scores are >= 0, so their bit patterns order like the floats.  A radix
 // select over four 8-bit digits finds the kblk-th largest key K and how
@@ -732,16 +795,20 @@ void launch_attn_prep(const AttnArgs& a, int nb, hipStream_t st) {
     else k_attn_prep<<<dim3((items + 3) / 4, nb), CHK_WG, 0, st>>>(a);
 }
 
-// Block keys, scores and selection; a no-op for rows still within the budget
-// (their block keys are still cached as blocks complete).
-void launch_qsa(const AttnArgs& a, int nb, hipStream_t st) {
-    if (!a.qsa) return;
+static void qsa_check(const AttnArgs& a) {
     // DPL = ihd / 64 dims per lane: 1, 2 or 4 (no 3-dim instantiation)
     if ((a.ihd != 64 && a.ihd != 128 && a.ihd != 256) || a.rot > 64 || a.rot > a.ihd || (a.rot & (a.rot - 1)) ||
         a.rot < 2 ||
         a.inh * a.ihd > 8 * 256 ||
         a.mask_words > QSA_MAX_WORDS || !a.iq_ready || !a.bscore || !a.vmask || !a.kv[0].block_k)
         throw std::runtime_error("QSA indexer shape not supported");
+}
+
+// Block keys, scores and selection; a no-op for rows still within the budget
+// (their block keys are still cached as blocks complete).
+void launch_qsa(const AttnArgs& a, int nb, hipStream_t st) {
+    if (!a.qsa) return;
+    qsa_check(a);
     const dim3 grid((a.max_blocks + QSA_BPG - 1) / QSA_BPG, nb);
     switch (a.ihd / 64) {
     case 1: k_qsa_score<1><<<grid, CHK_WG, 0, st>>>(a); break;
@@ -749,6 +816,23 @@ void launch_qsa(const AttnArgs& a, int nb, hipStream_t st) {
     default: k_qsa_score<4><<<grid, CHK_WG, 0, st>>>(a); break;
     }
     k_qsa_select<<<nb, QSA_SEL_WG, 0, st>>>(a);
+}
+
+void launch_pf_qsa(const AttnArgs& a, uint32_t nr, uint32_t nblk, hipStream_t st) {
+    qsa_check(a);
+    if (!nr) return;
+    // 16 rows of index queries and their padding
+    const uint32_t lds = a.inh * 4 * 16 * (a.ihd / 4 + 4) * 4;
+    if (lds > 65536) return launch_qsa(a, (int)nr, st);
+    if (nblk) {
+        const dim3 grid((nblk + QP_BLK - 1) / QP_BLK, (nr + 15) / 16);
+        switch (a.ihd / 64) {
+        case 1: k_pf_qsa_score<1><<<grid, CHK_WG, lds, st>>>(a, nr); break;
+        case 2: k_pf_qsa_score<2><<<grid, CHK_WG, lds, st>>>(a, nr); break;
+        default: k_pf_qsa_score<4><<<grid, CHK_WG, lds, st>>>(a, nr); break;
+        }
+    }
+    k_qsa_select<<<nr, QSA_SEL_WG, 0, st>>>(a);
 }
 
 void launch_qsa_block_keys(const AttnArgs& a, uint32_t blk0, uint32_t blk1, hipStream_t st) {

@@ -173,20 +173,20 @@ struct PfBufs {
     // the normed trunk streams, fc_e / fc_h outputs and the head's residual
     uint32_t* mtp_tok;
     float *mtp_en, *mtp_hn, *mtp_fe, *mtp_fh, *mtp_hyper;
-    // the flash attention plan (pf_flash_plan) for the chunk's dense rows,
-    // uploaded for the (rows, first position) key it was made for
+    // the flash attention plan (pf_flash_split) for the chunk's rows,
+    // uploaded for the (rows, first position) key it was made for (its
+    // partials take yd, free between an attention block's
+    // hyper-connection read and its out-projection)
     uint4 *fa_seg, *fa_merge;
-    float* fa_part;
     uint64_t fa_key = ~0ull;
     uint32_t fa_W = 0, fa_nslots = 0, fa_nmerge = 0;
-    // QSA past the budget: every row's index queries; scores, selections
-    // and attention partials of qsa_rows rows at a time
-    float *iq_ready, *qsa_bscore, *qsa_part;
-    uint32_t* qsa_vmask;
+    // QSA past the budget: every row's index queries; block scores of
+    // qsa_rows rows at a time
+    float *iq_ready, *qsa_bscore;
     uint32_t qsa_rows;
     // every row's block mask of the chunk's latest attention layer (rows
-    // that attend densely: no bits), for the debug_engine_blocks view;
-    // rows of the latest chunk
+    // that attend densely: no bits), which the flash kernel and the
+    // debug_engine_blocks view read; rows of the latest chunk
     uint32_t* qsa_rows_mask;
     uint32_t last_rows, last_pos0;
     // PLE over a chunk: table rows of each row's token, then as Scratch
@@ -1498,15 +1498,19 @@ struct ChkEngine {
     uint32_t prefill_rows_fit(bool all_logits) const;
     // ------------------------------------------------- GEMM prefill
     bool pf_supported() const;
-    // flash attention plans: workgroups per kv head, partial floats (at most
-    // two pieces per workgroup of a kv head)
-    uint64_t fa_wmax(uint64_t C) const {
-        return std::min<uint64_t>((C + 15) / 16, std::max<uint32_t>(1, ncu / D.nkv));
+    // flash attention plans: workgroups per kv head, segment and merge
+    // entries, partial slots (held in yd)
+    uint32_t fa_wmax(uint64_t C) const {
+        return (uint32_t)std::min<uint64_t>(8 * ((C + 15) / 16), std::max<uint32_t>(1, ncu / D.nkv));
     }
-    uint64_t fa_part_floats(uint64_t C) const { return (uint64_t)D.nkv * 2 * fa_wmax(C) * 16 * (D.nh / D.nkv) * (2 + D.hd); }
+    uint64_t fa_entries(uint64_t C) const { return std::max<uint64_t>((C + 15) / 16, fa_wmax(C)); }
+    uint64_t fa_slots(uint64_t C) const {
+        const uint32_t g = D.nh / D.nkv;
+        return C * (D.topk + 1) * D.H / ((uint64_t)D.nkv * pf_flash_rows(g) * g * (2 + D.hd));
+    }
     uint32_t pf_dense_rows(uint32_t T, uint32_t pos0) const;
     PfFlashLaunch pf_flash_launch(uint32_t T, uint32_t pos0);
-    uint32_t pf_qsa_rows() const;
+    uint32_t pf_qsa_rows(uint64_t C) const;
     void pf_alloc();
     void pf_hc_read(const HcDev& w, float* inj, uint32_t T, bool for_moe);
     void pf_out_proj(const Q4Mat& m, uint32_t K, uint32_t T);
@@ -1746,14 +1750,10 @@ uint64_t ChkEngine::prefill_scratch_bytes(uint64_t C, bool all_logits) const {
     if (D.SI != D.I) b += C * D.SI * f;
     if (dc_supported(D.nk, D.nv, D.dk, D.dv)) b += dc_work_floats((uint32_t)C, D.nv, D.dv) * f;
     if (all_logits) b += C * D.V * f;
-    {
-        const uint64_t rmax = (C + 15) / 16, wmax = fa_wmax(C);
-        b += (rmax * FA_MAXSEG + wmax) * 16 + fa_part_floats(C) * f;
-    }
+    b += fa_entries(C) * (FA_MAXSEG + 1) * 16;
     if (ple_l >= 0) b += C * (ngram_heads + c.ple_embed_dim + 3ull * D.hh + D.H) * 4;
     if (D.qsa)
-        b += (C * (D.inh * D.ihd + D.mask_words) +
-              (uint64_t)pf_qsa_rows() * (D.max_blocks + D.mask_words + (uint64_t)D.nh * max_chunks * (D.hd + 2))) * 4;
+        b += (C * (D.inh * D.ihd + D.mask_words) + (uint64_t)pf_qsa_rows(C) * D.max_blocks) * 4;
     return b;
 }
 
@@ -1788,13 +1788,14 @@ bool ChkEngine::pf_supported() const {
            (D.hd == 128 || D.hd == 256);
 }
 
-// Rows whose QSA selection and attention partials one prefill launch holds:
-// the partials of a row span every chunk of the context, so the group is
-// sized to about 256 MB of them (4..64 rows, a multiple of 4).
-uint32_t ChkEngine::pf_qsa_rows() const {
-    const uint64_t per_row = ((uint64_t)D.nh * max_chunks * (D.hd + 2) + D.max_blocks + D.mask_words) * 4;
-    const uint64_t fit = (256ull << 20) / std::max<uint64_t>(per_row, 1);
-    return (uint32_t)std::max<uint64_t>(4, std::min<uint64_t>(64, fit) / 4 * 4);
+// Rows whose QSA block scores one prefill launch holds: up to 64 MB of
+// them, and no more than the partials of 4..64 rows' attention over every
+// chunk of the context take (which bounds them for small contexts).
+uint32_t ChkEngine::pf_qsa_rows(uint64_t C) const {
+    const uint64_t per_row = ((uint64_t)D.nh * max_chunks * (D.hd + 2) + D.max_blocks) * 4;
+    const uint64_t rows = std::max<uint64_t>(4, std::min<uint64_t>(64, (256ull << 20) / std::max<uint64_t>(per_row, 1)) / 4 * 4);
+    const uint64_t fit = std::min<uint64_t>(64ull << 20, rows * per_row) / (4ull * D.max_blocks);
+    return (uint32_t)std::max<uint64_t>(1, std::min(C, fit));
 }
 
 void ChkEngine::pf_alloc() {
@@ -1834,9 +1835,8 @@ void ChkEngine::pf_alloc() {
     pf.inj_a = pfalloc<float>(C * D.hc);
     pf.inj_m = pfalloc<float>(C * D.hc);
     pf.mixed = pfalloc<float>(C * D.H);
-    pf.fa_seg = pfalloc<uint4>((C + 15) / 16 * FA_MAXSEG);
-    pf.fa_merge = pfalloc<uint4>(fa_wmax(C));
-    pf.fa_part = pfalloc<float>(fa_part_floats(C));
+    pf.fa_seg = pfalloc<uint4>(fa_entries(C) * FA_MAXSEG);
+    pf.fa_merge = pfalloc<uint4>(fa_entries(C));
     pf.fa_key = ~0ull;
     // DeltaNet / attention arena
     const uint64_t dn = C * (2ull * D.conv_dim + 2ull * D.v_dim + (2ull * pf_ab_split(D.H) + 2) * D.nv);
@@ -1878,12 +1878,10 @@ void ChkEngine::pf_alloc() {
     pf.yd = pfalloc<float>(C * slots * D.H);
     pf.dcw = dc_supported(D.nk, D.nv, D.dk, D.dv) ? pfalloc<float>(dc_work_floats((uint32_t)C, D.nv, D.dv)) : nullptr;
     if (D.qsa) {
-        pf.qsa_rows = pf_qsa_rows();
+        pf.qsa_rows = pf_qsa_rows(C);
         pf.iq_ready = pfalloc<float>(C * D.inh * D.ihd);
         pf.qsa_bscore = pfalloc<float>((uint64_t)pf.qsa_rows * D.max_blocks);
-        pf.qsa_vmask = pfalloc<uint32_t>((uint64_t)pf.qsa_rows * D.mask_words);
         pf.qsa_rows_mask = pfalloc<uint32_t>(C * D.mask_words);
-        pf.qsa_part = pfalloc<float>((uint64_t)pf.qsa_rows * D.nh * max_chunks * (D.hd + 2));
     }
     if (ple_l >= 0) {
         pf.ple_ids = pfalloc<uint32_t>(C * ngram_heads);
@@ -2112,50 +2110,40 @@ void ChkEngine::pf_attention(const LayerDev& L, uint32_t T, uint32_t pos0, const
     aa.theta = D.theta;
     aa.scale = D.attn_scale;
     aa.max_chunks = (pos0 + T - 1) / ATTN_CHUNK + 1;
+    PfFlashSel sel;
     if (!D.qsa) {
         launch_attn_prep(aa, (int)T, st);
-        launch_pf_flash(pf.q_ready, pf.q_raw, kvl, pf.attn_out, T, pos0, D.nh, D.nkv, D.hd, D.attn_scale,
-                        pf_flash_launch(T, pos0), st);
     } else {
         // select_tokens (cpu.rs:643-719) over the chunk: every row's KV,
         // index key and index queries first, then the pooled keys of the
         // blocks the chunk completes (later chunks and decode steps read
-        // them from block_k); rows still within the budget attend densely
-        // (the flash kernel), later rows through the decode path's block
-        // scores, top-kblk selection and masked partials, qsa_rows at a time
+        // them from block_k); rows past the budget have their blocks
+        // scored and the top kblk selected, qsa_rows at a time, and every
+        // row attends through the flash kernel under its selection
         set_qsa(aa, L);
         aa.iq_ready = pf.iq_ready;
         launch_attn_prep(aa, (int)T, st);
         launch_qsa_block_keys(aa, pos0 / D.ratio, (pos0 + T) / D.ratio, st);
         const uint32_t td = pf_dense_rows(T, pos0);
-        if (td) {
-            launch_pf_flash(pf.q_ready, pf.q_raw, kvl, pf.attn_out, td, pos0, D.nh, D.nkv, D.hd, D.attn_scale,
-                            pf_flash_launch(td, pos0), st);
-            launch_zero_f32(reinterpret_cast<float*>(pf.qsa_rows_mask), (uint64_t)td * D.mask_words, st);
-        }
+        if (td) launch_zero_f32(reinterpret_cast<float*>(pf.qsa_rows_mask), (uint64_t)td * D.mask_words, st);
         for (uint32_t r0 = td; r0 < T; r0 += pf.qsa_rows) {
             const uint32_t nr = std::min(pf.qsa_rows, T - r0);
             AttnArgs ag = aa;
-            ag.q_raw = pf.q_raw + (uint64_t)r0 * 2 * D.nh * D.hd;
-            ag.q_ready = pf.q_ready + (uint64_t)r0 * D.nh * D.hd;
             ag.iq_ready = pf.iq_ready + (uint64_t)r0 * D.inh * D.ihd;
             ag.pos = pf.pos + r0;
-            ag.out = pf.attn_out + (uint64_t)r0 * D.nh * D.hd;
             ag.bscore = pf.qsa_bscore;
-            ag.vmask = pf.qsa_vmask;
-            ag.part = pf.qsa_part;
-            ag.max_chunks = (pos0 + r0 + nr - 1) / ATTN_CHUNK + 1;
-            launch_qsa(ag, (int)nr, st);
-            launch_copy_f32(reinterpret_cast<float*>(pf.qsa_rows_mask) + (uint64_t)r0 * D.mask_words,
-                            reinterpret_cast<const float*>(pf.qsa_vmask), (uint64_t)nr * D.mask_words, st);
-            launch_attn_core(ag, (int)nr, st);
+            ag.vmask = pf.qsa_rows_mask + (uint64_t)r0 * D.mask_words;
+            launch_pf_qsa(ag, nr, (pos0 + r0 + nr) / D.ratio, st);
         }
+        if (td < T) sel = PfFlashSel{pf.qsa_rows_mask, D.mask_words, D.ratio, D.kblk};
     }
+    launch_pf_flash(pf.q_ready, pf.q_raw, kvl, pf.attn_out, T, pos0, D.nh, D.nkv, D.hd, D.attn_scale,
+                    pf_flash_launch(T, pos0), st, sel);
     launch_pf_xprep(pf.attn_out, D.nh * D.hd, T, D.nh * D.hd, pf.hi, pf.lo, pf.xs, st);
     pf_out_proj(L.at.o, D.nh * D.hd, T);
 }
 
-// Rows of a chunk that attend densely (the flash kernel): all of them, or
+// Rows of a chunk that attend densely: all of them, or
 // with QSA those before the first position whose blocks exceed the budget.
 uint32_t ChkEngine::pf_dense_rows(uint32_t T, uint32_t pos0) const {
     if (!D.qsa) return T;
@@ -2163,16 +2151,16 @@ uint32_t ChkEngine::pf_dense_rows(uint32_t T, uint32_t pos0) const {
     return first_sel <= pos0 ? 0 : std::min(T, first_sel - pos0);
 }
 
-// The flash plan for (T dense rows at pos0), made and uploaded when the key
+// The flash plan for (T rows at pos0), made and uploaded when the key
 // changes: at the start of a chunk, whose stream is then idle (the previous
 // chunk ended with a stream synchronisation); a change within a chunk waits
 // for the launches that may still read the old plan.
 PfFlashLaunch ChkEngine::pf_flash_launch(uint32_t T, uint32_t pos0) {
     const uint64_t key = (uint64_t)T << 32 | pos0;
     if (key != pf.fa_key) {
-        const PfFlashPlan p = pf_flash_split(T, pos0, (uint32_t)fa_wmax(pf.cap));
-        const uint64_t rmax = (pf.cap + 15) / 16, wmax = fa_wmax(pf.cap);
-        if (p.seg.size() > rmax * FA_MAXSEG || p.merge.size() > wmax || p.nslots > 2 * wmax)
+        const PfFlashPlan p = pf_flash_split(T, pos0, fa_wmax(pf.cap), pf_flash_rows(D.nh / D.nkv), fa_slots(pf.cap));
+        const uint64_t n = fa_entries(pf.cap);
+        if (p.seg.size() > n * FA_MAXSEG || p.merge.size() > n || p.nslots > fa_slots(pf.cap))
             throw std::runtime_error("flash attention plan exceeds its buffers");
         HIPCHK(hipStreamSynchronize(st));
         HIPCHK(hipMemcpy(pf.fa_seg, p.seg.data(), p.seg.size() * sizeof(uint4), hipMemcpyHostToDevice));
@@ -2183,7 +2171,7 @@ PfFlashLaunch ChkEngine::pf_flash_launch(uint32_t T, uint32_t pos0) {
         pf.fa_nslots = p.nslots;
         pf.fa_nmerge = (uint32_t)p.merge.size();
     }
-    return PfFlashLaunch{pf.fa_seg, pf.fa_merge, pf.fa_part, pf.fa_W, pf.fa_nslots, pf.fa_nmerge};
+    return PfFlashLaunch{pf.fa_seg, pf.fa_merge, pf.yd, pf.fa_W, pf.fa_nslots, pf.fa_nmerge};
 }
 
 // moe (cpu.rs:504-541) over the chunk: router GEMM, per-row top-k, entries
@@ -2312,7 +2300,7 @@ void ChkEngine::prefill_gemm(const uint32_t* toks, uint32_t n, uint32_t next_aft
         pf.moe_pend = nullptr;
         HIPCHK(hipMemsetAsync(pf.gcnt, 0, (D.E + 1) * PF_GCNT_STRIDE * 4, st));  // (and its expert counts)
         // the chunk's flash plan, while the stream is idle
-        if (const uint32_t td = pf_dense_rows(T, pos0)) pf_flash_launch(td, pos0);
+        pf_flash_launch(T, pos0);
         launch_pf_embed(pf.tokens, embed, pf.hyper, D.H, D.hc, T, st);
         for (uint32_t l = 0; l < c.num_hidden_layers; ++l) {
             const LayerDev& L = layers[l];
@@ -3343,12 +3331,12 @@ static int flash_plan_out(PfFlashPlan (*make)(uint32_t, uint32_t, uint32_t), uin
 
 int chk_pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
                       uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge) {
-    return flash_plan_out(pf_flash_plan, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
+    return flash_plan_out([](uint32_t t, uint32_t p, uint32_t w) { return pf_flash_plan(t, p, w); }, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
 }
 
 int chk_pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
                        uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge) {
-    return flash_plan_out(pf_flash_split, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
+    return flash_plan_out([](uint32_t t, uint32_t p, uint32_t w) { return pf_flash_split(t, p, w); }, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
 }
 
 int chk_copy_f32(float* dst, const float* src, uint64_t n, void* stream) {

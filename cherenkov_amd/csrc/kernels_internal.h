@@ -474,18 +474,27 @@ struct PfFlashPlan {
     std::vector<uint4> seg;    // [W][FA_MAXSEG]
     std::vector<uint4> merge;  // [split row blocks]
 };
-PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg);
+// rows of a row block: a workgroup's eight waves serve `g` query heads
+constexpr uint32_t pf_flash_rows(uint32_t g) { return g >= 8 ? 16u : 16u * (8u / g); }
+PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows = 16, bool whole_only = false);
 // the plan the engine takes: pf_flash_plan, or where the chunk has fewer row
-// blocks than max_wg, its steps over more workgroups than row blocks
-PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg);
+// blocks than max_wg, its steps over more workgroups than row blocks; at
+// most max_slots partial slots
+PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows = 16, uint64_t max_slots = ~0ull);
 struct PfFlashLaunch {         // a plan uploaded to the device
     const uint4* seg;
     const uint4* merge;
-    float* part;               // [nkv][nslots][16][nh / nkv][2 + hd]
+    float* part;               // [nkv][nslots][rows][nh / nkv][2 + hd]
     uint32_t W, nslots, nmerge;
 };
+// QSA: the rows' block selections (vmask null: every row attends densely)
+struct PfFlashSel {
+    const uint32_t* vmask = nullptr;  // [T][mask_words]
+    uint32_t mask_words = 0, ratio = 1, kblk = 0;
+};
 void launch_pf_flash(const float* q_ready, const float* q_raw, const KvDev& kv, float* out, uint32_t T, uint32_t pos0,
-                     uint32_t nh, uint32_t nkv, uint32_t hd, float scale, const PfFlashLaunch& plan, hipStream_t st);
+                     uint32_t nh, uint32_t nkv, uint32_t hd, float scale, const PfFlashLaunch& plan, hipStream_t st,
+                     const PfFlashSel& sel = PfFlashSel{});
 void launch_pf_gemm(const Q4Mat& w, const uint4* xhi, const uint4* xlo, const float* xs, float* y, uint32_t T,
                     uint32_t ldy, hipStream_t st);
 // [down; inject] partials -> inj and d, d staged as the up GEMM's operands
@@ -528,6 +537,9 @@ void launch_qsa_select(const AttnArgs& a, int nb, hipStream_t st);
 // block keys + scores + selection of nb rows (a no-op without QSA)
 void launch_qsa(const AttnArgs& a, int nb, hipStream_t st);
 // pooled keys of blocks [blk0, blk1) of kv[0]'s sequence
+// scores and selection of nr prefill rows (a.pos their positions, block keys
+// cached, at most nblk complete blocks) into a.bscore and a.vmask
+void launch_pf_qsa(const AttnArgs& a, uint32_t nr, uint32_t nblk, hipStream_t st);
 void launch_qsa_block_keys(const AttnArgs& a, uint32_t blk0, uint32_t blk1, hipStream_t st);
 void launch_attn_core(const AttnArgs& a, int nb, hipStream_t st);
 bool attn_shape_ok(uint32_t nh, uint32_t nkv, uint32_t hd);

@@ -2074,23 +2074,36 @@ namespace chk {
 // for every prompt row r at position pos0 + r and query head h,
 //   o = softmax_t(scale q . k_t) . v_t over t <= pos0 + r, times sigmoid(gate).
 //
-// Work: per kv head, (16-row block, 32-token tile) steps; row block rb
-// needs tiles 0 .. (pos0 + 16 rb + 15) / 32, so late blocks hold up to
-// twice the average.  A plan (pf_flash_plan, on the host) deals the steps
-// to the workgroups in equal shares: row blocks in zigzag order (first,
-// last, second, ...), the sequence cut into W equal ranges, so a workgroup
-// runs a few segments (row block, tile range); a row block cut between
-// workgroups leaves unnormalised partials (m, l, o) that k_pf_flash_join
-// joins.  Within a segment, wave w serves the kv head's query head w
-// (GQA: the group's waves share every staged K/V tile).  Per
-// 32-token tile the workgroup dequantises K and V (int8 x fp16 scale,
-// exact in f32) into LDS as fp16 hi + lo planes (V transposed), then each
-// wave runs S = Q K^T and O += P V on v_mfma_f32_16x16x32_f16 with three
-// passes (hi.hi + hi.lo + lo.hi, ~22-bit operands) and an online softmax in
-// f32.  Layouts (16x16x32): A lane l = row l%16, k (l/16)*8..+8; B lane l =
+// Work: per kv head, (row block, 32-token tile) steps; a row block is the
+// 16-row slices of the eight waves' rows (wave w: query head w % G of the
+// kv head, slice w / G, so every wave shares each staged K/V tile), and row
+// block rb needs the tiles up to its last row's position, so late blocks
+// hold up to twice the average.  A plan (pf_flash_split, on the host) deals
+// the steps to the workgroups in equal shares, so a workgroup runs a few
+// segments (row block, tile range); a row block cut between workgroups
+// leaves unnormalised partials (m, l, o) that k_pf_flash_join joins.
+//
+// Per tile the workgroup stages K as its int8 codes in fp16 (exact; one
+// plane) and V as int8 x fp16 scale (exact in f32) in fp16 hi + lo planes,
+// transposed.  Each wave runs S = Q K^T per 32-dim q8 block on
+// v_mfma_f32_16x16x32_f16 (q in hi + lo planes, two passes) with the
+// block's scale applied to the block's sums in f32, an online softmax in
+// f32, and O += P V in three passes (lo.hi + hi.lo + hi.hi, ~22-bit
+// operands).  The tile after the current one is stored while this one
+// computes (two LDS buffers, one barrier a tile), its raw bytes loaded a
+// tile earlier.  A wave holds its queries (64 registers) and outputs (64),
+// so a SIMD runs two waves and the step is latency-bound: per tile 1.1 us of
+// matrix unit, 1.4 us of vector unit and 1.2 us of LDS take 4.4 us.  2048
+// rows at position 0, 16 heads of 256 over 2: 180 + 19 us with both of K's
+// planes in LDS and one buffer, 156 + 14 so.
+// Layouts (16x16x32): A lane l = row l%16, k (l/16)*8..+8; B lane l =
 // column l%16, k (l/16)*8..+8; D lane l = column l%16, rows 4(l/16)..+4.
+//
+// SEL: QSA's selection (select_tokens, cpu.rs:643-719) as a mask: row r sees
+// token t when t's block of `ratio` tokens is in vmask's row r, past the
+// row's complete blocks, or the row has no more blocks than the budget.
 constexpr int FA_TOK = 32;    // tokens per staged tile
-constexpr int FA_ROWS = 16;   // query rows per workgroup
+constexpr int FA_ROWS = 16;   // query rows per wave
 
 struct PfFlashArgs {
     const float* q_ready;  // [T][nh][hd] normed, roped queries
@@ -2098,11 +2111,30 @@ struct PfFlashArgs {
     KvDev kv;
     float* out;            // [T][nh * hd]
     uint32_t T, pos0, nh, nkv;
-    float scale;
+    float scale2;          // the softmax scale times log2 e
     const uint4* seg;      // [W][FA_MAXSEG] the plan's segments (pf_flash_plan)
-    float* part;           // [nkv][nslots][FA_ROWS][G][2 + hd] partials of split row blocks
+    float* part;           // [nkv][nslots][rows][G][2 + hd] partials of split row blocks
     uint32_t nslots;
+    const uint32_t* vmask; // SEL: [T][mask_words] selected blocks
+    uint32_t mask_words, kblk;
+    float rratio;          // 1 / ratio
 };
+
+// the running maximum of a row that has seen no token: finite, far below any
+// score (which are sums of fp16-range products)
+constexpr float FA_LOWEST = -1.0e30f;
+
+// maximum over the 16 lanes of a DPP row, in every lane of it
+CHK_DEV float row_max16(float v) {
+    v = fmaxf(v, CHK_DPPF(v, 0xb1, 0xf, v));   // quad_perm [1,0,3,2]
+    v = fmaxf(v, CHK_DPPF(v, 0x4e, 0xf, v));   // quad_perm [2,3,0,1]
+    v = fmaxf(v, CHK_DPPF(v, 0x141, 0xf, v));  // row_half_mirror
+    return fmaxf(v, CHK_DPPF(v, 0x140, 0xf, v));  // row_mirror
+}
+
+// t / ratio for t < 2^20: t + 1/2 is exact and at least 1 / (2 t) of itself
+// away from the next quotient, far past the product's rounding
+CHK_DEV uint32_t fa_block(uint32_t t, float rratio) { return (uint32_t)(((float)t + 0.5f) * rratio); }
 
 CHK_DEV h8 split_hi(const float (&v)[8], h8& lo) {
     h8 hi;
@@ -2114,29 +2146,37 @@ CHK_DEV h8 split_hi(const float (&v)[8], h8& lo) {
     return hi;
 }
 
-template <int HD, int G>
-__global__ void __launch_bounds__(64 * G) k_pf_flash(PfFlashArgs a) {
-    constexpr int KS = HD / 32;          // dim steps of 32
+template <int HD, int G, bool SEL>
+__global__ void __launch_bounds__(512) k_pf_flash(PfFlashArgs a) {
+    constexpr int KS = HD / 32;          // dim steps of 32 (the q8 blocks)
     constexpr int DT = HD / 16;          // 16-dim output tiles
     constexpr int KP = HD + 8;           // padded K row (halves)
     constexpr int VP = FA_TOK + 8;       // padded V^T row (halves)
     constexpr int PP = FA_TOK + 8;       // padded P row (halves)
-    __shared__ __align__(16) _Float16 kh[FA_TOK][KP], kl[FA_TOK][KP];
-    __shared__ __align__(16) _Float16 vh[HD][VP], vl[HD][VP];
-    __shared__ __align__(16) _Float16 ph[G][FA_ROWS][PP], pl[G][FA_ROWS][PP];
-    constexpr uint32_t nthr = 64 * G;
-    constexpr int IPT = (FA_TOK * HD / 16 + nthr - 1) / nthr;  // staging items per thread
-    const uint32_t tid = threadIdx.x, lane = tid & 63, w = wave_id();
-    const uint32_t col = lane & 15, kq = lane >> 4;
-    const uint32_t hk = blockIdx.y, h = hk * G + w;
+    constexpr int NW = 8, ROWS = FA_ROWS * (NW / G);
+    __shared__ __align__(16) _Float16 kc[2][FA_TOK][KP];
+    __shared__ __align__(16) float ksc[2][FA_TOK][KS];
+    __shared__ __align__(16) _Float16 vh[2][HD][VP], vl[2][HD][VP];
+    __shared__ __align__(16) _Float16 ph[NW][FA_ROWS][PP], pl[NW][FA_ROWS][PP];
+    constexpr uint32_t nthr = 64 * NW;
+    static_assert(FA_TOK * HD / 16 <= (int)nthr, "one staging item per thread");
+    const uint32_t w = wave_id();
+    const uint32_t hk = blockIdx.y, h = hk * G + w % G;
     const uint32_t kv_row = a.nkv * HD, last_tok = a.pos0 + a.T - 1;
+    const int8_t *kbase = a.kv.k + hk * HD, *vbase = a.kv.v + hk * HD;
+    const uint16_t *ksbase = a.kv.ks + hk * (HD / 32), *vsbase = a.kv.vs + hk * (HD / 32);
     const uint4* segs = a.seg + (size_t)blockIdx.x * FA_MAXSEG;
     for (uint32_t sgi = 0; sgi < FA_MAXSEG; ++sgi) {
     const uint4 sg = segs[sgi];  // (row block, first tile, end tile, slot or ~0: the whole block)
     if (sg.x == ~0u) break;
+    // (opaque per segment: addresses formed from the thread id are rebuilt
+    // where they are used, not kept in registers across the tile loop)
+    uint32_t tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const uint32_t lane = tid & 63, col = lane & 15, kq = lane >> 4;
     if (sgi) __syncthreads();  // every wave is done with the previous segment's tiles
     const uint32_t rb = sg.x, ta = sg.y, tb = sg.z;
-    const uint32_t r0 = rb * FA_ROWS;
+    const uint32_t r0 = rb * ROWS + (w / G) * FA_ROWS;
     // this wave's queries as A operands
     h8 qh[KS], ql[KS];
     {
@@ -2148,130 +2188,207 @@ __global__ void __launch_bounds__(64 * G) k_pf_flash(PfFlashArgs a) {
             const float4 v1 = *reinterpret_cast<const float4*>(qp + s * 32 + kq * 8 + 4);
             const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
             qh[s] = split_hi(v, ql[s]);
+            if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
     }
-    // positions of the 4 rows this lane holds in D layout (rows past T
-    // repeat the last row; they are never written)
-    uint32_t qpos[4];
+    // position of the first of the 4 rows this lane holds in D layout (rows
+    // past T hold the last row's queries; they are never written)
+    const uint32_t qp0 = a.pos0 + r0 + kq * 4;
+    uint32_t nblk[4], mrow[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) qpos[i] = a.pos0 + min(r0 + kq * 4 + i, a.T - 1);
+    for (int i = 0; i < 4; ++i) {
+        nblk[i] = 0;
+        if (SEL) {
+            // complete blocks of a row past the budget; a dense row has none to select
+            const uint32_t n = fa_block(qp0 + i + 1, a.rratio);
+            nblk[i] = n > a.kblk ? n : 0;
+            mrow[i] = min(qp0 + i - a.pos0, a.T - 1) * a.mask_words;
+        }
+    }
     f4 o[DT];
 #pragma unroll
     for (int d = 0; d < DT; ++d) o[d] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     float m[4], l[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        m[i] = -INFINITY;
+        m[i] = FA_LOWEST;
         l[i] = 0.0f;
     }
     // Staging: K as (token tid % 32, 16 dims), V as (token pair tid % 16,
     // 8 dims) so that the transposed V writes are whole dwords in
-    // consecutive banks; a tile's raw bytes are loaded one tile ahead.
-    uint4 kraw[IPT];
-    uint2 vraw[IPT][2];
-    uint16_t ksc[IPT], vsc[IPT][2];
+    // consecutive banks.
+    uint4 kraw = make_uint4(0, 0, 0, 0);
+    uint2 vraw[2];
+    uint16_t kscr = 0, vscr[2];
+    uint32_t mw[2][4] = {};  // SEL: the mask words of this lane's 2 tokens x 4 rows
+    const bool live = tid < (uint32_t)(FA_TOK * HD / 16);
+    const uint32_t skt = tid % FA_TOK, skd = (tid / FA_TOK) * 16;
+    const uint32_t svt = 2 * (tid % (FA_TOK / 2)), svd = (tid / (FA_TOK / 2)) * 8;
     auto load_raw = [&](uint32_t t0) __attribute__((always_inline)) {
+        // (tokens past the last repeat it: masked below, and finite)
+        if (live) {
+            const uint32_t kt = min(t0 + skt, last_tok);
+            // (32-bit offsets: a cache plane is at most 2^18 tokens x 2^13 bytes)
+            kraw = *reinterpret_cast<const uint4*>(kbase + (kt * kv_row + skd));
+            kscr = ksbase[kt * (kv_row / 32) + skd / 32];
 #pragma unroll
-        for (int r = 0; r < IPT; ++r) {
-            const uint32_t i = tid + r * nthr;
-            kraw[r] = make_uint4(0, 0, 0, 0);
-            vraw[r][0] = vraw[r][1] = make_uint2(0, 0);
-            ksc[r] = vsc[r][0] = vsc[r][1] = 0;
-            if (i >= (uint32_t)(FA_TOK * HD / 16)) continue;
-            const uint32_t kt = t0 + i % FA_TOK, kd = (i / FA_TOK) * 16;
-            if (kt <= last_tok) {
-                kraw[r] = *reinterpret_cast<const uint4*>(a.kv.k + (size_t)kt * kv_row + hk * HD + kd);
-                ksc[r] = a.kv.ks[(size_t)kt * (kv_row / 32) + (hk * HD + kd) / 32];
+            for (int e = 0; e < 2; ++e) {
+                const uint32_t vt = min(t0 + svt + e, last_tok);
+                vraw[e] = *reinterpret_cast<const uint2*>(vbase + (vt * kv_row + svd));
+                vscr[e] = vsbase[vt * (kv_row / 32) + svd / 32];
             }
-            const uint32_t vt = t0 + 2 * (i % (FA_TOK / 2)), vd = (i / (FA_TOK / 2)) * 8;
-#pragma unroll
-            for (int e = 0; e < 2; ++e)
-                if (vt + e <= last_tok) {
-                    vraw[r][e] = *reinterpret_cast<const uint2*>(a.kv.v + (size_t)(vt + e) * kv_row + hk * HD + vd);
-                    vsc[r][e] = a.kv.vs[(size_t)(vt + e) * (kv_row / 32) + (hk * HD + vd) / 32];
-                }
         }
     };
-    auto store_tile = [&]() __attribute__((always_inline)) {
+    // the tile's visibility as 8 bits (4 tt + i), from the words load_mask brought
+    auto visible = [&](uint32_t t0) __attribute__((always_inline)) -> uint32_t {
+        uint32_t vb = 0;
 #pragma unroll
-        for (int r = 0; r < IPT; ++r) {
-            const uint32_t i = tid + r * nthr;
-            if (i >= (uint32_t)(FA_TOK * HD / 16)) continue;
-            const uint32_t kt = i % FA_TOK, kd = (i / FA_TOK) * 16;
-            const float kscale = __half2float(__ushort_as_half(ksc[r]));
-            const uint32_t kwv[4] = {kraw[r].x, kraw[r].y, kraw[r].z, kraw[r].w};
+        for (int tt = 0; tt < 2; ++tt) {
+            const uint32_t t = t0 + tt * 16 + col, blk = SEL ? fa_block(t, a.rratio) : 0;
 #pragma unroll
-            for (int hlf = 0; hlf < 2; ++hlf) {
-                float kv8[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    kv8[j] = (float)(int8_t)(kwv[hlf * 2 + j / 4] >> (8 * (j % 4))) * kscale;
-                h8 lo8;
-                const h8 hi8 = split_hi(kv8, lo8);
-                *reinterpret_cast<h8*>(&kh[kt][kd + hlf * 8]) = hi8;
-                *reinterpret_cast<h8*>(&kl[kt][kd + hlf * 8]) = lo8;
+            for (int i = 0; i < 4; ++i) {
+                bool v = t <= qp0 + i;
+                if (SEL) v = v && (blk >= nblk[i] || ((mw[tt][i] >> (blk & 31)) & 1u));
+                vb |= v ? 1u << (4 * tt + i) : 0u;
             }
-            const uint32_t vt = 2 * (i % (FA_TOK / 2)), vd = (i / (FA_TOK / 2)) * 8;
-            const float vs0 = __half2float(__ushort_as_half(vsc[r][0])), vs1 = __half2float(__ushort_as_half(vsc[r][1]));
-            const uint32_t v0[2] = {vraw[r][0].x, vraw[r][0].y}, v1[2] = {vraw[r][1].x, vraw[r][1].y};
+        }
+        return vb;
+    };
+    auto load_mask = [&](uint32_t t0) __attribute__((always_inline)) {
+        if (!SEL) return;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float x0 = (float)(int8_t)(v0[j / 4] >> (8 * (j % 4))) * vs0;
-                const float x1 = (float)(int8_t)(v1[j / 4] >> (8 * (j % 4))) * vs1;
-                const _Float16 h0 = (_Float16)x0, h1 = (_Float16)x1;
-                typedef _Float16 hh2 __attribute__((ext_vector_type(2)));
-                *reinterpret_cast<hh2*>(&vh[vd + j][vt]) = hh2{h0, h1};
-                *reinterpret_cast<hh2*>(&vl[vd + j][vt]) = hh2{(_Float16)(x0 - (float)h0), (_Float16)(x1 - (float)h1)};
-            }
+        for (int tt = 0; tt < 2; ++tt) {
+            const uint32_t wd = min(fa_block(t0 + tt * 16 + col, a.rratio) >> 5, a.mask_words - 1);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mw[tt][i] = a.vmask[(size_t)(mrow[i] + wd)];
+        }
+    };
+    auto store_tile = [&](uint32_t buf) __attribute__((always_inline)) {
+        if (!live) return;
+        // the codes + 128 as bytes of fp16 1024 + v, less 1152: exact
+        typedef _Float16 hh2 __attribute__((ext_vector_type(2)));
+        const uint32_t kwv[4] = {kraw.x ^ 0x80808080u, kraw.y ^ 0x80808080u, kraw.z ^ 0x80808080u, kraw.w ^ 0x80808080u};
+        const hh2 off = {(_Float16)1152.0f, (_Float16)1152.0f};
+        uint32_t kp[8];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, kwv[q], 0x04010400u);
+            const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, kwv[q], 0x04030402u);
+            kp[2 * q] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(hh2, lo) - off);
+            kp[2 * q + 1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(hh2, hi) - off);
+        }
+        *reinterpret_cast<uint4*>(&kc[buf][skt][skd]) = make_uint4(kp[0], kp[1], kp[2], kp[3]);
+        *reinterpret_cast<uint4*>(&kc[buf][skt][skd + 8]) = make_uint4(kp[4], kp[5], kp[6], kp[7]);
+        if ((skd & 16) == 0) ksc[buf][skt][skd / 32] = __half2float(__ushort_as_half(kscr));
+        // V of the token pair, packed: hi = fp16(code * scale) and the exact
+        // remainder (the product has 19 bits and no bit below the scale's)
+        const hh2 vs = __builtin_bit_cast(hh2, (uint32_t)vscr[0] | (uint32_t)vscr[1] << 16);
+        // (every other 32 threads take their dims 4..7 first: in the same
+        // order, lanes 32..63 would write the banks of lanes 0..31)
+        const bool sw = tid & 32;
+        const uint32_t v0[2] = {(sw ? vraw[0].y : vraw[0].x) ^ 0x80808080u, (sw ? vraw[0].x : vraw[0].y) ^ 0x80808080u};
+        const uint32_t v1[2] = {(sw ? vraw[1].y : vraw[1].x) ^ 0x80808080u, (sw ? vraw[1].x : vraw[1].y) ^ 0x80808080u};
+        const uint32_t vd = svd + (sw ? 4 : 0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t sel = 0x0c000c00u | (uint32_t)(j % 4) | (uint32_t)(4 + j % 4) << 16;
+            const uint32_t pr = __builtin_amdgcn_perm(v1[j / 4], v0[j / 4], sel) | 0x64006400u;
+            const hh2 c = __builtin_bit_cast(hh2, pr) - off;
+            const hh2 hi = c * vs;
+            const uint32_t row = j < 4 ? vd + j : (vd ^ 4) + (j - 4);  // svd % 8 = 0
+            *reinterpret_cast<hh2*>(&vh[buf][row][svt]) = hi;
+            *reinterpret_cast<hh2*>(&vl[buf][row][svt]) = __builtin_elementwise_fma(c, vs, -hi);
         }
     };
     load_raw(ta * FA_TOK);
-    store_tile();
+    load_mask(ta * FA_TOK);
+    store_tile(0);
+    if (ta + 1 < tb) load_raw((ta + 1) * FA_TOK);
     __syncthreads();
     for (uint32_t tile = ta; tile < tb; ++tile) {
-        const uint32_t t0 = tile * FA_TOK;
-        if (tile + 1 < tb) load_raw(t0 + FA_TOK);
-        // ---- S = Q K^T for 2 token tiles
+        const uint32_t t0 = tile * FA_TOK, buf = (tile - ta) & 1;
+        // the next tile into the other buffer (read by nobody since the last
+        // barrier), the one after that requested
+        if (tile + 1 < tb) {
+            store_tile(buf ^ 1);
+            if (tile + 2 < tb) load_raw(t0 + 2 * FA_TOK);
+        }
+        const uint32_t vb = SEL ? visible(t0) : 0;
+        __builtin_amdgcn_sched_barrier(0);  // (phases kept apart: their registers together spill)
+        // ---- S = Q K^T for 2 token tiles, block sums times the key's block
+        // scale (the operand of step n + QD is requested before step n's products)
         f4 s[2];
+        constexpr int QD = 4, QN = 2 * KS;
+        h8 fk[QD + 1];
+        float4 sc[2][KS / 4];
+        auto kfrag = [&](int n) __attribute__((always_inline)) -> h8 {
+            return *reinterpret_cast<const h8*>(&kc[buf][(n / KS) * 16 + col][(n % KS) * 32 + kq * 8]);
+        };
+#pragma unroll
+        for (int n = 0; n < QD; ++n) fk[n] = kfrag(n);
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt) {
             s[tt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const h8 bh = *reinterpret_cast<const h8*>(&kh[tt * 16 + col][ks * 32 + kq * 8]);
-                const h8 bl = *reinterpret_cast<const h8*>(&kl[tt * 16 + col][ks * 32 + kq * 8]);
-                s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ql[ks], bh, s[tt], 0, 0, 0);
-                s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[ks], bl, s[tt], 0, 0, 0);
-                s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[ks], bh, s[tt], 0, 0, 0);
-            }
+            for (int q = 0; q < KS / 4; ++q) sc[tt][q] = *reinterpret_cast<const float4*>(&ksc[buf][tt * 16 + col][q * 4]);
+        }
+#pragma unroll
+        for (int n = 0; n < QN; ++n) {
+            const int tt = n / KS, ks = n % KS;
+            if (n + QD < QN) fk[(n + QD) % (QD + 1)] = kfrag(n + QD);
+            const h8 bk = fk[n % (QD + 1)];
+            f4 pt = __builtin_amdgcn_mfma_f32_16x16x32_f16(ql[ks], bk, f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+            pt = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[ks], bk, pt, 0, 0, 0);
+            const float4 s4 = sc[tt][ks / 4];
+            const float sv = ks % 4 == 0 ? s4.x : ks % 4 == 1 ? s4.y : ks % 4 == 2 ? s4.z : s4.w;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[tt][i] = fmaf(sv, pt[i], s[tt][i]);
+            if (n % 2 == 1) __builtin_amdgcn_sched_barrier(0);
         }
         // ---- online softmax over the tile (rows kq*4 + i, tokens col, 16 + col)
-        float p[2][4];
+        float p[2][4], mn[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            float mx = -INFINITY;
+            float mx = FA_LOWEST;
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt) {
-                const uint32_t t = t0 + tt * 16 + col;
-                const float v = t <= qpos[i] ? s[tt][i] * a.scale : -INFINITY;
+                const bool vis = SEL ? (vb >> (4 * tt + i)) & 1u : t0 + tt * 16 + col <= qp0 + i;
+                const float v = vis ? s[tt][i] * a.scale2 : -INFINITY;
                 p[tt][i] = v;
                 mx = fmaxf(mx, v);
             }
-            mx = group_max<16>(mx);
-            const float mn = fmaxf(m[i], mx);
-            const float corr = m[i] == -INFINITY ? 0.0f : expf(m[i] - mn);
+            mx = row_max16(mx);
+            mn[i] = fmaxf(m[i], mx);
+        }
+        // (in base 2; m starts at the lowest finite value, so that a row
+        // without a visible token so far keeps finite differences)
+        if (__any(mn[0] > m[0] || mn[1] > m[1] || mn[2] > m[2] || mn[3] > m[3])) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float corr = __builtin_amdgcn_exp2f(m[i] - mn[i]);
+                l[i] *= corr;
+                m[i] = mn[i];
+#pragma unroll
+                for (int d = 0; d < DT; ++d) o[d][i] *= corr;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
             float rs = 0.0f;
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt) {
-                const float e = p[tt][i] == -INFINITY ? 0.0f : expf(p[tt][i] - mn);
-                p[tt][i] = e;
-                rs += e;
+                p[tt][i] = __builtin_amdgcn_exp2f(p[tt][i] - m[i]);
+                rs += p[tt][i];
             }
-            rs = group_sum<16>(rs);
-            l[i] = l[i] * corr + rs;
-            m[i] = mn;
+            l[i] += group_sum<16>(rs);
+        }
+        if (tile + 1 < tb) load_mask(t0 + FA_TOK);
+        constexpr int PD = 2;
+        h8 fh[PD + 1], fl[PD + 1];
 #pragma unroll
-            for (int d = 0; d < DT; ++d) o[d][i] *= corr;
+        for (int d = 0; d < PD; ++d) {
+            fh[d] = *reinterpret_cast<const h8*>(&vh[buf][d * 16 + col][kq * 8]);
+            fl[d] = *reinterpret_cast<const h8*>(&vl[buf][d * 16 + col][kq * 8]);
         }
         // ---- P to this wave's LDS rows (hi, lo), read back as A operands:
         // LDS instructions of one wave complete in order, so only the
@@ -2291,110 +2408,144 @@ __global__ void __launch_bounds__(64 * G) k_pf_flash(PfFlashArgs a) {
         const h8 pal = *reinterpret_cast<const h8*>(&pl[w][col][kq * 8]);
 #pragma unroll
         for (int d = 0; d < DT; ++d) {
-            const h8 bh = *reinterpret_cast<const h8*>(&vh[d * 16 + col][kq * 8]);
-            const h8 bl = *reinterpret_cast<const h8*>(&vl[d * 16 + col][kq * 8]);
+            // (the operands of step d + PD are requested before step d's products)
+            if (d + PD < DT) {
+                fh[(d + PD) % (PD + 1)] = *reinterpret_cast<const h8*>(&vh[buf][(d + PD) * 16 + col][kq * 8]);
+                fl[(d + PD) % (PD + 1)] = *reinterpret_cast<const h8*>(&vl[buf][(d + PD) * 16 + col][kq * 8]);
+            }
+            const h8 bh = fh[d % (PD + 1)], bl = fl[d % (PD + 1)];
             o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pal, bh, o[d], 0, 0, 0);
             o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pah, bl, o[d], 0, 0, 0);
             o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pah, bh, o[d], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if (tile + 1 < tb) {
-            __syncthreads();  // every wave is done with this tile's K and V
-            store_tile();
-            __syncthreads();
-        }
+        if (tile + 1 < tb) __syncthreads();  // the next tile is staged, this one read
     }
+    uint32_t el = threadIdx.x & 63;
+    asm volatile("" : "+v"(el));
+    const uint32_t ecol = el & 15, ekq = el >> 4;
     if (sg.w == ~0u) {
         // ---- o / l times the per-dim sigmoid gate (cpu.rs:629-633)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const uint32_t r = r0 + kq * 4 + i;
+            const uint32_t r = r0 + ekq * 4 + i;
             if (r >= a.T) continue;
             const float inv = 1.0f / l[i];
             const float* gp = a.q_raw + ((size_t)r * a.nh + h) * 2 * HD + HD;
             float* op = a.out + (size_t)r * a.nh * HD + (size_t)h * HD;
 #pragma unroll
             for (int d = 0; d < DT; ++d) {
-                const uint32_t dd = d * 16 + col;
+                const uint32_t dd = d * 16 + ecol;
                 op[dd] = o[d][i] * inv * sigmoidf_(gp[dd]);
             }
         }
     } else {
         // ---- a piece of a split row block: (m, l, unnormalised o) per row
-        float* pp = a.part + ((size_t)hk * a.nslots + sg.w) * FA_ROWS * G * (2 + HD);
+        float* pp = a.part + ((size_t)hk * a.nslots + sg.w) * ROWS * G * (2 + HD);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            float* q = pp + ((size_t)(kq * 4 + i) * G + w) * (2 + HD);
-            if (col == 0) {
+            float* q = pp + ((size_t)((w / G) * FA_ROWS + ekq * 4 + i) * G + w % G) * (2 + HD);
+            if (ecol == 0) {
                 q[0] = m[i];
                 q[1] = l[i];
             }
 #pragma unroll
-            for (int d = 0; d < DT; ++d) q[2 + d * 16 + col] = o[d][i];
+            for (int d = 0; d < DT; ++d) q[2 + d * 16 + ecol] = o[d][i];
         }
     }
     }
 }
 
 // Joins the pieces of the row blocks a flash plan split: per row, head and
-// dim, o = sum_k o_k e^(m_k - M) / sum_k l_k e^(m_k - M) with M = max_k m_k
-// (a piece whose tokens a row cannot see holds m = -inf, l = 0), times the
-// sigmoid gate.  Workgroup (entry, row, query head); the pieces' weights
-// e^(m_k - M) / L meet in LDS (np <= FA_MAXJOIN), then thread d sums dim d
-// over the pieces, eight loads in flight.
-__global__ void __launch_bounds__(256) k_pf_flash_join(PfFlashArgs a, const uint4* __restrict__ merge, uint32_t G,
-                                                       uint32_t hd) {
-    __shared__ float sm[FA_MAXJOIN], red[8];
+// dim, o = sum_k o_k 2^(m_k - M) / sum_k l_k 2^(m_k - M) with M = max_k m_k
+// (a piece whose tokens a row cannot see holds m = FA_LOWEST, l = 0), times the
+// sigmoid gate.  A wave per (entry, row of gridDim.y, query head), four
+// heads a workgroup: lane k holds the weights of pieces k, k + 64, ... (np
+// <= FA_MAXJOIN), lane d sums dims DPL d .. + DPL, four pieces in flight.
+template <int DPL>
+__global__ void __launch_bounds__(256) k_pf_flash_join(PfFlashArgs a, const uint4* __restrict__ merge, uint32_t G) {
+    constexpr uint32_t HD = 64 * DPL, NK = FA_MAXJOIN / 64;
+    typedef float fd __attribute__((ext_vector_type(2)));
     const uint4 me = merge[blockIdx.x];  // (row block, first slot, pieces, 0)
-    const uint32_t row = blockIdx.y, hk = blockIdx.z / G, g = blockIdx.z % G, t = threadIdx.x;
-    const uint32_t r = me.x * FA_ROWS + row, np = me.z;
-    if (r >= a.T) return;
-    const size_t ps = (size_t)FA_ROWS * G * (2 + hd);  // floats per slot
-    const float* __restrict__ p0 = a.part + ((size_t)hk * a.nslots + me.y) * ps + ((size_t)row * G + g) * (2 + hd);
-    const uint32_t h = hk * G + g, dc = min(t, hd - 1);
-    const float gate = a.q_raw[((size_t)r * a.nh + h) * 2 * hd + hd + dc];
-    float m = -INFINITY, l = 0.0f;
-    if (t < np) {
-        m = p0[t * ps];
-        l = p0[t * ps + 1];
+    const uint32_t row = blockIdx.y, h = blockIdx.z * 4 + wave_id(), lane = threadIdx.x & 63;
+    const uint32_t r = me.x * gridDim.y + row, np = me.z;
+    if (r >= a.T || h >= a.nh) return;
+    const uint32_t hk = h / G, g = h % G;
+    const size_t ps = (size_t)gridDim.y * G * (2 + HD);  // floats per slot
+    const float* __restrict__ p0 = a.part + ((size_t)hk * a.nslots + me.y) * ps + ((size_t)row * G + g) * (2 + HD);
+    fd gate[DPL / 2];
+    const fd* gp = reinterpret_cast<const fd*>(a.q_raw + ((size_t)r * a.nh + h) * 2 * HD + HD + lane * DPL);
+#pragma unroll
+    for (int j = 0; j < DPL / 2; ++j) gate[j] = gp[j];
+    const float* __restrict__ po = p0 + 2 + lane * DPL;
+    auto piece = [&](uint32_t k, fd (&v)[DPL / 2]) __attribute__((always_inline)) {
+        const fd* q = reinterpret_cast<const fd*>(po + min(k, np - 1) * ps);
+#pragma unroll
+        for (int j = 0; j < DPL / 2; ++j) v[j] = q[j];
+    };
+    fd v[4][DPL / 2];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) piece(k, v[k]);
+    float m[NK], l[NK], M = FA_LOWEST, L = 0.0f;
+#pragma unroll
+    for (uint32_t i = 0; i < NK; ++i) {
+        m[i] = FA_LOWEST;
+        l[i] = 0.0f;
+        if (64 * i < np) {
+            const uint32_t k = lane + 64 * i;
+            const fd ml = *reinterpret_cast<const fd*>(p0 + min(k, np - 1) * ps);
+            if (k < np) {
+                m[i] = ml.x;
+                l[i] = ml.y;
+            }
+        }
+        M = fmaxf(M, m[i]);
     }
-    const float M = block_max(m, red);
-    const float e = m == -INFINITY ? 0.0f : expf(m - M);
-    const float L = block_sum(l * e, red);
-    if (t < np) sm[t] = e;
-    __syncthreads();
-    const float* __restrict__ po = p0 + 2 + dc;
-    float O = 0.0f;
-    uint32_t k = 0;
-    for (; k + 8 <= np; k += 8) {
-        float v[8];
+    M = wave_max(M);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = po[(k + j) * ps];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) O += v[j] * sm[k + j];
+    for (uint32_t i = 0; i < NK; ++i) {
+        m[i] = __builtin_amdgcn_exp2f(m[i] - M);
+        L += l[i] * m[i];
     }
-    {
-        float v[8];
+    L = wave_sum(L);
+    float O[DPL] = {};
+    for (uint32_t k0 = 0; k0 < np; k0 += 4) {
+        fd u[4][DPL / 2];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = po[min(k + j, np - 1) * ps];
+        for (int k = 0; k < 4; ++k) piece(k0 + 4 + k, u[k]);  // (past the last: re-read)
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-            if (k + j < np) O += v[j] * sm[k + j];
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t kk = min(k0 + k, np - 1), i = kk >> 6;
+            const float ms = i == 0 ? m[0] : i == 1 ? m[1] : i == 2 ? m[2] : m[3];
+            float e = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ms), (int)(kk & 63)));
+            if (k0 + k >= np) e = 0.0f;
+#pragma unroll
+            for (int j = 0; j < DPL; ++j) O[j] += v[k][j / 2][j % 2] * e;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int j = 0; j < DPL / 2; ++j) v[k][j] = u[k][j];
     }
-    if (t < hd) a.out[(size_t)r * a.nh * hd + (size_t)h * hd + t] = O * (1.0f / L) * sigmoidf_(gate);
+    const float inv = 1.0f / L;
+    fd* op = reinterpret_cast<fd*>(a.out + ((size_t)r * a.nh + h) * HD + lane * DPL);
+#pragma unroll
+    for (int j = 0; j < DPL / 2; ++j)
+        op[j] = fd{O[2 * j] * inv * sigmoidf_(gate[j].x), O[2 * j + 1] * inv * sigmoidf_(gate[j].y)};
 }
 
 // Deals every kv head's (row block, tile) steps to max_wg workgroups in
 // equal shares (see k_pf_flash); one whole row block per workgroup, heavy
 // ones first, where the blocks' work is within 15% of even or a share
 // would need more than FA_MAXSEG segments.
-PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg) {
+PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows, bool whole_only) {
     PfFlashPlan p;
-    const uint32_t R = (T + FA_ROWS - 1) / FA_ROWS;
+    const uint32_t R = (T + rows - 1) / rows;
     std::vector<uint32_t> tiles(R);
     uint64_t total = 0;
     uint32_t most = 0;
     for (uint32_t rb = 0; rb < R; ++rb) {
-        tiles[rb] = (pos0 + std::min(rb * FA_ROWS + FA_ROWS - 1, T - 1)) / FA_TOK + 1;
+        tiles[rb] = (pos0 + std::min(rb * rows + rows - 1, T - 1)) / FA_TOK + 1;
         total += tiles[rb];
         most = std::max(most, tiles[rb]);
     }
@@ -2409,7 +2560,7 @@ PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg) {
         }
         return p;
     };
-    if ((double)most <= 1.15 * (double)total / W) return whole();
+    if (whole_only || (double)most <= 1.15 * (double)total / W) return whole();
     p.W = W;
     p.seg.assign((size_t)W * FA_MAXSEG, make_uint4(~0u, 0, 0, 0));
     std::vector<uint32_t> order;
@@ -2454,14 +2605,19 @@ PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg) {
 // workgroups: 673 us a layer, against 48 split + 8 to join; 333 behind 1500:
 // 264 -> 67 + 12.
 // A range costs its queries and its partial once, about two tiles' time.
-PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg) {
-    const uint32_t R = (T + FA_ROWS - 1) / FA_ROWS;
+PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows, uint64_t max_slots) {
+    const uint32_t R = (T + rows - 1) / rows;
     std::vector<uint64_t> first(R + 1, 0);
     for (uint32_t rb = 0; rb < R; ++rb)
-        first[rb + 1] = first[rb] + (pos0 + std::min(rb * FA_ROWS + FA_ROWS - 1, T - 1)) / FA_TOK + 1;
+        first[rb + 1] = first[rb] + (pos0 + std::min(rb * rows + rows - 1, T - 1)) / FA_TOK + 1;
     const uint64_t total = first[R];
-    const uint32_t W = (uint32_t)std::min<uint64_t>({max_wg, total / FA_MINSHARE, (uint64_t)FA_MAXJOIN - 1});
-    if (R >= max_wg || W <= R) return pf_flash_plan(T, pos0, max_wg);
+    const uint32_t W = (uint32_t)std::min<uint64_t>(
+        {max_wg, total / FA_MINSHARE, (uint64_t)FA_MAXJOIN - 1, max_slots > R ? max_slots - R : 0});
+    auto even = [&]() {
+        PfFlashPlan p = pf_flash_plan(T, pos0, max_wg, rows);
+        return p.nslots <= max_slots ? p : pf_flash_plan(T, pos0, R, rows, true);
+    };
+    if (R >= max_wg || W <= R) return even();
     PfFlashPlan p;
     p.W = W;
     p.seg.assign((size_t)W * FA_MAXSEG, make_uint4(~0u, 0, 0, 0));
@@ -2476,7 +2632,7 @@ PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg) {
         for (; k < W && k * total / W < first[rb + 1]; ++k) {
             const uint64_t lo = std::max(first[rb], k * total / W), hi = std::min(first[rb + 1], (k + 1) * total / W);
             if (lo >= hi) continue;
-            if (nseg[k] == FA_MAXSEG) return pf_flash_plan(T, pos0, max_wg);
+            if (nseg[k] == FA_MAXSEG) return even();
             p.seg[(size_t)k * FA_MAXSEG + nseg[k]++] =
                 make_uint4(rb, (uint32_t)(lo - first[rb]), (uint32_t)(hi - first[rb]), split ? p.nslots++ : ~0u);
         }
@@ -2486,31 +2642,36 @@ PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg) {
 }
 
 void launch_pf_flash(const float* q_ready, const float* q_raw, const KvDev& kv, float* out, uint32_t T, uint32_t pos0,
-                     uint32_t nh, uint32_t nkv, uint32_t hd, float scale, const PfFlashLaunch& plan, hipStream_t st) {
+                     uint32_t nh, uint32_t nkv, uint32_t hd, float scale, const PfFlashLaunch& plan, hipStream_t st,
+                     const PfFlashSel& sel) {
     if (nkv == 0 || nh % nkv || nh / nkv > 8 || (hd != 128 && hd != 256))
         throw std::runtime_error("flash prefill takes head_dim 128 or 256 and up to 8 query heads per kv head");
     if (!T) return;
     if (!plan.seg || !plan.W || (plan.nmerge && (!plan.merge || !plan.part)))
         throw std::runtime_error("flash prefill needs its plan");
-    PfFlashArgs a{q_ready, q_raw, kv, out, T, pos0, nh, nkv, scale, plan.seg, plan.part, plan.nslots};
+    PfFlashArgs a{q_ready, q_raw, kv, out, T, pos0, nh, nkv, scale * 1.44269504088896341f, plan.seg, plan.part, plan.nslots,
+                  sel.vmask, sel.mask_words, sel.kblk, 1.0f / (float)sel.ratio};
     const dim3 grid(plan.W, nkv);
-#define CHK_FA(HDV)                                                                                      \
-    switch (nh / nkv) {                                                                                  \
-    case 1: k_pf_flash<HDV, 1><<<grid, 64, 0, st>>>(a); break;                                           \
-    case 2: k_pf_flash<HDV, 2><<<grid, 128, 0, st>>>(a); break;                                          \
-    case 3: case 4: k_pf_flash<HDV, 4><<<grid, 256, 0, st>>>(a); break;                                  \
-    default: k_pf_flash<HDV, 8><<<grid, 512, 0, st>>>(a); break;                                         \
-    }
-    if (nh / nkv != 1 && nh / nkv != 2 && nh / nkv != 4 && nh / nkv != 8)
+    const uint32_t g = nh / nkv;
+    if (g != 1 && g != 2 && g != 4 && g != 8)
         throw std::runtime_error("flash prefill takes 1, 2, 4 or 8 query heads per kv head");
+#define CHK_FA(HDV, SELV)                                                        \
+    switch (g) {                                                                 \
+    case 1: k_pf_flash<HDV, 1, SELV><<<grid, 512, 0, st>>>(a); break;            \
+    case 2: k_pf_flash<HDV, 2, SELV><<<grid, 512, 0, st>>>(a); break;            \
+    case 4: k_pf_flash<HDV, 4, SELV><<<grid, 512, 0, st>>>(a); break;            \
+    default: k_pf_flash<HDV, 8, SELV><<<grid, 512, 0, st>>>(a); break;           \
+    }
     if (hd == 256) {
-        CHK_FA(256)
+        if (sel.vmask) { CHK_FA(256, true) } else { CHK_FA(256, false) }
     } else {
-        CHK_FA(128)
+        if (sel.vmask) { CHK_FA(128, true) } else { CHK_FA(128, false) }
     }
 #undef CHK_FA
-    if (plan.nmerge)
-        k_pf_flash_join<<<dim3(plan.nmerge, FA_ROWS, nh), CHK_WG, 0, st>>>(a, plan.merge, nh / nkv, hd);
+    if (!plan.nmerge) return;
+    const dim3 jgrid(plan.nmerge, pf_flash_rows(g), (nh + 3) / 4);
+    if (hd == 256) k_pf_flash_join<4><<<jgrid, CHK_WG, 0, st>>>(a, plan.merge, g);
+    else k_pf_flash_join<2><<<jgrid, CHK_WG, 0, st>>>(a, plan.merge, g);
 }
 
 }  // namespace chk
