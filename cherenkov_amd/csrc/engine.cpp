@@ -1513,6 +1513,7 @@ struct ChkEngine {
     uint32_t pf_qsa_rows(uint64_t C) const;
     void pf_alloc();
     void pf_hc_read(const HcDev& w, float* inj, uint32_t T, bool for_moe);
+    void pf_in_proj(const PfGemmArgs& g, uint32_t T);
     void pf_out_proj(const Q4Mat& m, uint32_t K, uint32_t T);
     void pf_deltanet(const LayerDev& L, uint32_t T);
     void pf_attention(const LayerDev& L, uint32_t T, uint32_t pos0, const KvDev* kvo = nullptr);
@@ -1745,7 +1746,7 @@ uint64_t ChkEngine::prefill_scratch_bytes(uint64_t C, bool all_logits) const {
     b += std::max(dn, at) * f;
     b += C * (PF_ROUTER_CHUNKS * D.E + 1 + 2ull * D.topk) * f + (D.E + 1ull) * C * 4 +
          (PF_GCNT_STRIDE + 1ull) * (D.E + 1) * 4;
-    b += (uint64_t)(pf_tile_bound((uint32_t)C, D.topk, D.E, 48) + pf_tile_bound((uint32_t)C, D.topk, D.E, 64)) * 12 +
+    b += (uint64_t)(pf_tile_bound((uint32_t)C, D.topk, D.E, 32)) * 12 +
          C * slots * (D.I + D.H) * f + C * slots * 4 + (D.E + 1) * 4;
     if (D.SI != D.I) b += C * D.SI * f;
     if (dc_supported(D.nk, D.nv, D.dk, D.dv)) b += dc_work_floats((uint32_t)C, D.nv, D.dv) * f;
@@ -1868,11 +1869,11 @@ void ChkEngine::pf_alloc() {
     pf.count = pfalloc<uint32_t>(D.E + 1);
     pf.gcnt = pfalloc<uint32_t>((D.E + 1) * PF_GCNT_STRIDE);
     HIPCHK(hipMemset(pf.gcnt, 0, (D.E + 1) * PF_GCNT_STRIDE * 4));
-    pf.tiles = pfalloc<uint32_t>(pf_tile_bound((uint32_t)C, D.topk, D.E, 48) + pf_tile_bound((uint32_t)C, D.topk, D.E, 64));
-    pf.tinfo = pfalloc<uint2>(pf_tile_bound((uint32_t)C, D.topk, D.E, 48) + pf_tile_bound((uint32_t)C, D.topk, D.E, 64));
+    pf.tiles = pfalloc<uint32_t>(pf_tile_bound((uint32_t)C, D.topk, D.E, 32));
+    pf.tinfo = pfalloc<uint2>(pf_tile_bound((uint32_t)C, D.topk, D.E, 32));
     pf.goff = pfalloc<uint32_t>(D.E + 1);
     pf.gpos = pfalloc<uint32_t>(C * slots);
-    pf.ntiles = pfalloc<uint32_t>(2);
+    pf.ntiles = pfalloc<uint32_t>(1);
     pf.act = pfalloc<float>(C * slots * D.I);
     pf.act_sh = D.SI != D.I ? pfalloc<float>(C * D.SI) : nullptr;
     pf.yd = pfalloc<float>(C * slots * D.H);
@@ -1911,22 +1912,27 @@ void ChkEngine::pf_hc_read(const HcDev& w, float* inj, uint32_t T, bool for_moe)
                       (uint64_t)pf.cap * D.H, pf.pend_split, pf.inj_a, st, mc);
     pf.pend = nullptr;
     // [down; inject] is narrow (lowrank + hc outputs) over a long K = hc H:
-    // split K by stream, partials summed in stream order by the finisher
+    // split K by stream, a few rows' further (as far as the partials fit),
+    // partials summed in K order by the finisher
     const uint32_t N = D.lowrank + D.hc;
+    // (the partials' buffer holds hc chunks of a full chunk's rows; the
+    // expert activations' f32 rows, free here, more at most shapes)
+    const uint64_t act_fit = (uint64_t)pf.cap * (D.topk + 1) * D.I / ((uint64_t)T * N), own_fit = (uint64_t)pf.cap * D.hc / T;
+    float* part = act_fit > own_fit ? pf.act : pf.hc_part;
     PfGemmArgs g{};
-    g.seg[0] = PfSeg{w.down, pf.hc_part, N, 0};
-    g.seg[1] = PfSeg{w.inject, pf.hc_part + D.lowrank, N, D.lowrank};
+    g.seg[0] = PfSeg{w.down, part, N, 0};
+    g.seg[1] = PfSeg{w.inject, part + D.lowrank, N, D.lowrank};
     g.nseg = 2;
     g.N = N;
     g.K = D.hh;
     g.M = T;
-    g.ksplit = D.hc;
+    g.ksplit = pf_ksplit(N, D.hh, T, D.hc, (uint32_t)std::min<uint64_t>(16, std::max(act_fit, own_fit)));
     g.zstride = (uint64_t)T * N;
     g.xhi = pf.hi;
     g.xlo = pf.lo;
     g.xs = pf.xs;
     launch_pf_gemm_args(g, PE_STORE, mt, st);
-    launch_pf_hc_down_finish(pf.hc_part, D.hc, T, D.lowrank, D.hc, 1.0f / (float)D.hc, pf.d, inj, pf.dhi, pf.dlo, pf.dxs,
+    launch_pf_hc_down_finish(part, g.ksplit, T, D.lowrank, D.hc, 1.0f / (float)D.hc, pf.d, inj, pf.dhi, pf.dlo, pf.dxs,
                              st);
     PfGemmArgs u{};
     u.seg[0].m = w.up;
@@ -1975,9 +1981,10 @@ void ChkEngine::pf_hc_read(const HcDev& w, float* inj, uint32_t T, bool for_moe)
 // A block's out-projection (K inputs -> H) over the chunk's staged
 // operands.  Its inject into the hc streams (cpu.rs:971-979) is left to the
 // next hyper-connection read, which reads and rewrites every stream anyway:
-// the GEMM stores K-chunk partials (two chunks: twice the workgroups of a
-// one-pass launch, whose 8 column blocks x 64-row tiles gave the CUs one
-// workgroup each) into yd, free until the expert down projection.
+// the GEMM stores K-chunk partials (two chunks at 2048 rows: twice the
+// workgroups of a one-pass launch, whose 8 column blocks x 64-row tiles gave
+// the CUs one workgroup each; up to eight at fewer rows) into yd, free until
+// the expert down projection.
 void ChkEngine::pf_out_proj(const Q4Mat& m, uint32_t K, uint32_t T) {
     if (pf.pend) throw std::runtime_error("an out-projection is already pending");
     pf_moe_flush();  // (its partials take yd)
@@ -1988,7 +1995,7 @@ void ChkEngine::pf_out_proj(const Q4Mat& m, uint32_t K, uint32_t T) {
     o.N = D.H;
     o.K = K;
     o.M = T;
-    o.ksplit = G % 2 == 0 && (G / 2) % 8 == 0 ? 2 : 1;
+    o.ksplit = G % 2 == 0 && (G / 2) % 8 == 0 ? pf_ksplit(D.H, K, T, 2, std::min<uint32_t>(8, D.topk + 1)) : 1;
     o.zstride = (uint64_t)pf.cap * D.H;
     o.xhi = pf.hi;
     o.xlo = pf.lo;
@@ -1996,6 +2003,27 @@ void ChkEngine::pf_out_proj(const Q4Mat& m, uint32_t K, uint32_t T) {
     launch_pf_gemm_args(o, PE_STORE, (T + 63) / 64, st);
     pf.pend = pf.yd;
     pf.pend_split = o.ksplit;
+}
+
+// A mixer's input projections (segments of g, over the staged rows).  Few
+// rows leave CUs idle: K then goes over up to four chunks, whose partials
+// (in yd, free here) one pass sums into the segments.
+void ChkEngine::pf_in_proj(const PfGemmArgs& g, uint32_t T) {
+    const uint64_t fit = (uint64_t)pf.cap * (D.topk + 1) * D.H / ((uint64_t)T * g.N);
+    const uint32_t ks = pf_ksplit(g.N, g.K, T, 1, (uint32_t)std::min<uint64_t>(4, fit), 2);
+    if (ks < 4 || g.N % 4) {
+        launch_pf_gemm_args(g, PE_STORE, (T + 63) / 64, st);
+        return;
+    }
+    PfGemmArgs p = g;
+    for (uint32_t q = 0; q < g.nseg; ++q) {
+        p.seg[q].y = pf.yd + g.seg[q].n0;
+        p.seg[q].ldy = g.N;
+    }
+    p.ksplit = ks;
+    p.zstride = (uint64_t)T * g.N;
+    launch_pf_gemm_args(p, PE_STORE, (T + 63) / 64, st);
+    launch_pf_sum_parts(g, pf.yd, ks, T, st);
 }
 
 // linear_attention (cpu.rs:745-826) over the chunk: the qkv and z input
@@ -2015,7 +2043,7 @@ void ChkEngine::pf_deltanet(const LayerDev& L, uint32_t T) {
     g.xhi = pf.hi;
     g.xlo = pf.lo;
     g.xs = pf.xs;
-    launch_pf_gemm_args(g, PE_STORE, mt, st);
+    pf_in_proj(g, T);
     // a and b (2 nv outputs): as 64 more columns of the GEMM above they made
     // a last column block of workgroups, a whole extra pass over the CUs
     // at the 80B shape; split K, their workgroups are short
@@ -2087,7 +2115,7 @@ void ChkEngine::pf_attention(const LayerDev& L, uint32_t T, uint32_t pos0, const
     g.xhi = pf.hi;
     g.xlo = pf.lo;
     g.xs = pf.xs;
-    launch_pf_gemm_args(g, PE_STORE, mt, st);
+    pf_in_proj(g, T);
     AttnArgs aa{};
     aa.q_raw = pf.q_raw;
     aa.k_raw = pf.k_raw;
@@ -2221,13 +2249,10 @@ void ChkEngine::pf_moe(const LayerDev& L, uint32_t T) {
     dn.xhi = pf.ahi;
     dn.xlo = pf.alo;
     dn.xs = pf.axs;
-    // experts hold from one row to over a thousand (T k / E on average):
-    // both GEMMs take 64-row tiles, whose empty 16-row slices the kernel
-    // skips
-    const uint32_t tr = 64;
-    dn.tiles = pf.tiles + pf_tile_bound(T, D.topk, D.E, tr);
-    dn.tinfo = pf.tinfo + pf_tile_bound(T, D.topk, D.E, tr);
-    dn.ntiles = pf.ntiles + 1;
+    // experts hold from one row to over a thousand (T k / E on average);
+    // a tile's empty 16-row slices are skipped
+    const uint32_t tr = pf_tile_rows(gu, dn, T, D.topk, D.E);
+    gu.trows = dn.trows = tr;
     // (also counts the layer's expert activity)
     launch_pf_group(pf.gcnt, T, D.topk, D.E, pf.cap, pf.count, pf.tiles, pf.ntiles, pf.tinfo, pf.goff, act,
                     L.moe.record_layer, tr, shared_grouped, st);
@@ -2251,7 +2276,7 @@ void ChkEngine::pf_moe(const LayerDev& L, uint32_t T) {
         launch_pf_gemm_args(sh, PE_SILU_MUL, (T + 63) / 64, st);
     }
     if (!staged) launch_pf_xprep(pf.act, D.I, T * slots, D.I, pf.ahi, pf.alo, pf.axs, st);
-    launch_pf_gemm_args(dn, PE_STORE, pf_tile_bound(T, D.topk, D.E, 64), st);
+    launch_pf_gemm_args(dn, PE_STORE, pf_tile_bound(T, D.topk, D.E, tr), st);
     if (!shared_grouped) {
         // token t's shared slot of yd: grouped row T k + t, after the routed rows
         launch_pf_xprep(pf.act_sh, D.SI, T, D.SI, pf.hi, pf.lo, pf.xs, st);

@@ -330,6 +330,7 @@ struct PfGemmArgs {
     const uint2* tinfo;      // per tile: (group's first row in grouped order, group's row count)
     const uint32_t* ntiles;
     uint32_t cap, div;
+    uint32_t trows;          // rows of a tile of the list: 64, or 32 (staged scales)
     ExpertsDev X;            // routed-expert records for groups < X.experts
     ExpertsDev X4;           // their 4-bit copies, for records whose kind is 0
     const uint8_t* kinds;    // [record layers][experts] with a low-bit X (else null)
@@ -495,6 +496,9 @@ struct PfFlashSel {
 void launch_pf_flash(const float* q_ready, const float* q_raw, const KvDev& kv, float* out, uint32_t T, uint32_t pos0,
                      uint32_t nh, uint32_t nkv, uint32_t hd, float scale, const PfFlashLaunch& plan, hipStream_t st,
                      const PfFlashSel& sel = PfFlashSel{});
+uint32_t pf_tile_rows(const PfGemmArgs& gate_up, const PfGemmArgs& down, uint32_t T, uint32_t topk, uint32_t E);
+void launch_pf_sum_parts(const PfGemmArgs& a, const float* part, uint32_t nsplit, uint32_t T, hipStream_t st);
+uint32_t pf_ksplit(uint32_t N, uint32_t K, uint32_t T, uint32_t least, uint32_t most, uint32_t per_cu = 1);
 void launch_pf_gemm(const Q4Mat& w, const uint4* xhi, const uint4* xlo, const float* xs, float* y, uint32_t T,
                     uint32_t ldy, hipStream_t st);
 // [down; inject] partials -> inj and d, d staged as the up GEMM's operands

@@ -199,12 +199,24 @@ __global__ void __launch_bounds__(256) k_pf_hc_prep(float* __restrict__ hyper, c
             const uint32_t kb = min(tau + 256 * j, bps - 1);
 #pragma unroll
             for (int e = 0; e < 8; ++e) pv[j][e] = 0.0f;
-            for (uint32_t z = 0; z < nsplit; ++z) {
-                const float4* p = reinterpret_cast<const float4*>(part + z * pzs + (size_t)t * H + kb * 8);
-                const float4 u0 = p[0], u1 = p[1];
-                const float w8[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+            // two partials' loads in flight (past the last: re-read, not added)
+            for (uint32_t z0 = 0; z0 < nsplit; z0 += 2) {
+                float4 u[2][2];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) pv[j][e] += w8[e];
+                for (int z = 0; z < 2; ++z) {
+                    const float4* p =
+                        reinterpret_cast<const float4*>(part + min(z0 + z, nsplit - 1) * pzs + (size_t)t * H + kb * 8);
+                    u[z][0] = p[0];
+                    u[z][1] = p[1];
+                }
+#pragma unroll
+                for (int z = 0; z < 2; ++z) {
+                    const float w8[8] = {u[z][0].x, u[z][0].y, u[z][0].z, u[z][0].w,
+                                         u[z][1].x, u[z][1].y, u[z][1].z, u[z][1].w};
+                    if (z0 + z < nsplit)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) pv[j][e] += w8[e];
+                }
             }
         }
     }
@@ -309,6 +321,7 @@ __global__ void __launch_bounds__(256) k_pf_hc_prep(float* __restrict__ hyper, c
 // 16 outputs: mixed = (1/hc) sum_g sigmoid(v_g) normed_g, cpu.rs:477-491),
 // PE_SILU_MUL (NMAT 2: silu(gate) * up, mlp, cpu.rs:981-992).
 constexpr int PF_WG = 256;  // threads per GEMM workgroup
+constexpr uint32_t PF_CUS = 256;  // compute units the launch rules count on
 constexpr int PF_AROW = 9;  // uint4 per staged A row (8 + 1 pad: bank spread)
 
 CHK_DEV h8 pf_unpack(uint32_t w, const Q4Consts& qk) {
@@ -337,7 +350,7 @@ CHK_DEV h8 pf_unpack(uint32_t w, const Q4Consts& qk) {
 // midpoint rule (step s, half s + b), folded per lane in f32, so such
 // launches run without staged scales.
 template <int NMAT, int EPI, bool SBL, int BITS = 4, int NI = 4>
-__global__ void __launch_bounds__(PF_WG, 2) k_pf_gemm(PfGemmArgs ka) {
+__global__ void __launch_bounds__(PF_WG, NI < 4 ? 3 : 2) k_pf_gemm(PfGemmArgs ka) {
     // The arguments read through the kernarg segment's own (constant)
     // address space: every use is then a scalar load at its point of use
     // rather than a value held in SGPRs across the kernel (the kernel's
@@ -364,7 +377,7 @@ __global__ void __launch_bounds__(PF_WG, 2) k_pf_gemm(PfGemmArgs ka) {
     // scales it folds are 4 consecutive staged rows and its results leave
     // as 16-byte stores straight from registers
     constexpr bool SW = SBL;
-    __shared__ __align__(16) u32x4 sA[2][2][64 * PF_AROW];
+    __shared__ __align__(16) u32x4 sA[2][2][TR * PF_AROW];
     __shared__ __align__(16) float sX[2][64];
     __shared__ __align__(16) float sSB[SBL ? 2 : 1][SBL ? 8 * 256 : 1];  // [block][group % 8][local row]
     __shared__ uint32_t sRow[64];  // Y row of each tile row (staged epilogue)
@@ -473,12 +486,12 @@ __global__ void __launch_bounds__(PF_WG, 2) k_pf_gemm(PfGemmArgs ka) {
         offs(q, row_of(wn_, j, rem & 15), ow, ld_so, ob);
     }
 
-    // ---- A staging: thread tid loads 8-blocks 2 (tid % 4) + {0, 1} of row
-    // tid / 4 (hi, lo planes) and the group sum of row tid % 64
-    // (tiles under 64 rows: the threads past the tile re-read its last row,
-    // into buffer rows nobody reads; no branch keeps the pipeline's
-    // registers in one straight schedule)
-    const uint32_t lrow = tid >> 2, lkb = (tid & 3) * 2;
+    // ---- A staging: NI pieces (8-blocks of one plane) a thread.  64-row
+    // tiles: 8-blocks 2 (tid % 4) + {0, 1} of row tid / 4, both planes;
+    // 32-row tiles: 8-block tid % 8 of row tid / 8, both planes.
+    static_assert(NI == 4 || NI == 2, "tiles of 64 or 32 rows");
+    const uint32_t lrow = NI == 4 ? tid >> 2 : tid >> 3;
+    const uint32_t lkb = NI == 4 ? (tid & 3) * 2 : tid & 7;
     uint32_t arow_ld, arow_xs;
     {
         const uint32_t m = min(m0 + min(lrow, TR - 1), M - 1);
@@ -496,17 +509,21 @@ __global__ void __launch_bounds__(PF_WG, 2) k_pf_gemm(PfGemmArgs ka) {
     // unconditional (past the last group it re-reads the last one), so the
     // wait counters the compiler derives stay exact: a step waits only for
     // the loads it consumes.
-    u32x4 rah0[2], rah1[2], ral0[2], ral1[2];
+    u32x4 ra[2][NI];  // NI 4: hi 0, hi 1, lo 0, lo 1; NI 2: hi, lo
     float rx[2];
     u32x2 bw[2][NMAT][NJ];                         // words 2 kq, 2 kq + 1: K-steps 0, 1
     uint16_t bs[2][SBL ? 1 : NMAT][SBL ? 1 : NJ];  // per-lane scale, bias (not SBL)
     uint16_t bb[2][SBL ? 1 : NMAT][SBL ? 1 : NJ];
     u32x4 sreg_s;                                  // SBL: the next block's 8 scales
     auto fetch = [&](int slot, uint32_t g) __attribute__((always_inline)) {
-        rah0[slot] = ghi[g * 8];
-        rah1[slot] = ghi[g * 8 + 1];
-        ral0[slot] = glo[g * 8];
-        ral1[slot] = glo[g * 8 + 1];
+        ra[slot][0] = ghi[g * 8];
+        if constexpr (NI == 4) {
+            ra[slot][1] = ghi[g * 8 + 1];
+            ra[slot][2] = glo[g * 8];
+            ra[slot][3] = glo[g * 8 + 1];
+        } else {
+            ra[slot][1] = glo[g * 8];
+        }
         if (!SBL) rx[slot] = gxs[g];
 #pragma unroll
         for (int q = 0; q < NMAT; ++q)
@@ -530,10 +547,14 @@ __global__ void __launch_bounds__(PF_WG, 2) k_pf_gemm(PfGemmArgs ka) {
             }
     };
     auto a_store = [&](int slot, uint32_t buf) __attribute__((always_inline)) {
-        sA[buf][0][lrow * PF_AROW + lkb] = rah0[slot];
-        sA[buf][0][lrow * PF_AROW + lkb + 1] = rah1[slot];
-        sA[buf][1][lrow * PF_AROW + lkb] = ral0[slot];
-        sA[buf][1][lrow * PF_AROW + lkb + 1] = ral1[slot];
+        sA[buf][0][lrow * PF_AROW + lkb] = ra[slot][0];
+        if constexpr (NI == 4) {
+            sA[buf][0][lrow * PF_AROW + lkb + 1] = ra[slot][1];
+            sA[buf][1][lrow * PF_AROW + lkb] = ra[slot][2];
+            sA[buf][1][lrow * PF_AROW + lkb + 1] = ra[slot][3];
+        } else {
+            sA[buf][1][lrow * PF_AROW + lkb] = ra[slot][1];
+        }
         if (!SBL) sX[buf][tid & 63] = rx[slot];  // four identical writes per row: no branch
     };
     auto sb_fetch = [&](uint32_t g0) __attribute__((always_inline)) {
@@ -1213,18 +1234,36 @@ __global__ void __launch_bounds__(256) k_pf_hc_down_finish_q(const float* __rest
         if (j >= (uint64_t)T * hc) return;
         const uint32_t t = (uint32_t)(j / hc), g = (uint32_t)(j % hc);
         float v = 0.0f;
-        for (uint32_t z = 0; z < nsplit; ++z) v += part[z * zstride + (size_t)t * N + lowrank + g];
+        for (uint32_t z0 = 0; z0 < nsplit; z0 += 4) {
+            float u[4];
+#pragma unroll
+            for (uint32_t z = 0; z < 4; ++z) u[z] = part[min(z0 + z, nsplit - 1) * zstride + (size_t)t * N + lowrank + g];
+#pragma unroll
+            for (uint32_t z = 0; z < 4; ++z)
+                if (z0 + z < nsplit) v += u[z];
+        }
         v *= alpha;
         inj[(size_t)t * hc + g] = 2.0f * sigmoidf_(v);
         return;
     }
     const uint32_t t = (uint32_t)(i / blocks), kb = (uint32_t)(i % blocks);
     float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t z = 0; z < nsplit; ++z) {
-        const float4* p = reinterpret_cast<const float4*>(part + z * zstride + (size_t)t * N + kb * 8);
-        const float4 u0 = p[0], u1 = p[1];
-        v[0] += u0.x; v[1] += u0.y; v[2] += u0.z; v[3] += u0.w;
-        v[4] += u1.x; v[5] += u1.y; v[6] += u1.z; v[7] += u1.w;
+    // four partials' loads in flight (past the last: re-read, not added)
+    for (uint32_t z0 = 0; z0 < nsplit; z0 += 4) {
+        float4 u[4][2];
+#pragma unroll
+        for (uint32_t z = 0; z < 4; ++z) {
+            const float4* p =
+                reinterpret_cast<const float4*>(part + min(z0 + z, nsplit - 1) * zstride + (size_t)t * N + kb * 8);
+            u[z][0] = p[0];
+            u[z][1] = p[1];
+        }
+#pragma unroll
+        for (uint32_t z = 0; z < 4; ++z)
+            if (z0 + z < nsplit) {
+                v[0] += u[z][0].x; v[1] += u[z][0].y; v[2] += u[z][0].z; v[3] += u[z][0].w;
+                v[4] += u[z][1].x; v[5] += u[z][1].y; v[6] += u[z][1].z; v[7] += u[z][1].w;
+            }
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = siluf_(v[j] * alpha);
@@ -1243,6 +1282,29 @@ __global__ void __launch_bounds__(256) k_pf_hc_down_finish_q(const float* __rest
     hi[i] = __builtin_bit_cast(uint4, h);
     lo[i] = __builtin_bit_cast(uint4, l);
     if ((kb & 7) == 0) xs[(size_t)t * (lowrank >> 6) + (kb >> 3)] = s;
+}
+
+// K-chunk partials [nsplit][T][N] of a projection summed in chunk order into
+// its segments' outputs: a thread takes four outputs of a row (segments
+// start and end on a multiple of four).
+__global__ void __launch_bounds__(256) k_pf_sum_parts(PfGemmArgs a, const float* __restrict__ part, uint32_t nsplit,
+                                                      uint32_t T) {
+    const uint32_t n = (blockIdx.x * CHK_WG + threadIdx.x) * 4, t = blockIdx.y;
+    if (n >= a.N) return;
+    const float4* p = reinterpret_cast<const float4*>(part + (size_t)t * a.N + n);
+    const size_t zs = (size_t)T * a.N / 4;
+    float4 u[4];
+#pragma unroll
+    for (uint32_t z = 0; z < 4; ++z) u[z] = p[min(z, nsplit - 1) * zs];
+    float4 v = u[0];
+#pragma unroll
+    for (uint32_t z = 1; z < 4; ++z)
+        if (z < nsplit) v = make_float4(v.x + u[z].x, v.y + u[z].y, v.z + u[z].z, v.w + u[z].w);
+    PfSeg s = a.seg[0];
+#pragma unroll
+    for (uint32_t q = 1; q < 4; ++q)
+        if (q < a.nseg && n >= a.seg[q].n0) s = a.seg[q];
+    *reinterpret_cast<float4*>(s.y + (size_t)t * s.ldy + (n - s.n0)) = v;
 }
 
 // ------------------------------------------------------------- router
@@ -1443,9 +1505,6 @@ __global__ void __launch_bounds__(256) k_pf_route(const float* __restrict__ logi
 // them: first every group of two or more tiles, its count rounded up to
 // even (the extra tile has no rows), so each starts at an even position
 // (the GEMMs run tiles 2c and 2c + 1 on one XCD), then the one-tile groups.
-// A second such list of 64-row tiles follows at tiles + pf_tile_bound(T,
-// topk, E, tr), ntiles[1] of them (the gate/up and down GEMMs tile the same
-// entries differently).
 // Per tile also tinfo[] = (the group's first row in grouped order, its row
 // count), per group goff[] = that first row, and per entry pos[] = its
 // group << 22 | its place in the group (grouped row goff[group] + place;
@@ -1462,7 +1521,7 @@ __global__ void __launch_bounds__(PG_WG) k_pf_group(uint32_t* __restrict__ gcnt,
                                                     uint32_t* __restrict__ tiles, uint32_t* __restrict__ ntiles,
                                                     uint2* __restrict__ tinfo, uint32_t* __restrict__ goff,
                                                     unsigned long long* __restrict__ act, uint32_t layer,
-                                                    uint32_t tr, uint32_t topk, uint32_t shared) {
+                                                    uint32_t tr, uint32_t shared) {
     __shared__ uint32_t cnt[PG_WG];
     __shared__ uint32_t offs[PG_WG];
     __shared__ unsigned long long wsum[PG_WG / 64];
@@ -1495,49 +1554,38 @@ __global__ void __launch_bounds__(PG_WG) k_pf_group(uint32_t* __restrict__ gcnt,
         ae[0] += cnt[e];
         ae[1] += 1;
     }
-    // one tile list per tile height: tr-row tiles at tiles, 64-row tiles
-    // at tiles + pf_tile_bound(T, topk, E, tr) (*ntiles, ntiles[1] of
-    // them).  Tiles come in five classes, in this order: the tiles of the
-    // longer groups, then the one-tile groups by their 16-row slices, most
-    // first (the GEMMs deal workgroups in list order, so a launch ends on
-    // its shortest ones); per group a count in the 12-bit field of its
-    // class of one 64-bit workgroup prefix sum (the launcher keeps the
-    // counts under 4096).
-    const uint32_t trs[2] = {tr, 64u};
-    uint32_t* dst = tiles;
+    // Tiles come in five classes, in this order: the tiles of the longer
+    // groups, then the one-tile groups by their 16-row slices, most first
+    // (the GEMMs deal workgroups in list order, so a launch ends on its
+    // shortest ones); per group a count in the 12-bit field of its class of
+    // one 64-bit workgroup prefix sum (the launcher keeps the counts under
+    // 4096).
     auto field = [](unsigned long long v, uint32_t k) { return (uint32_t)(v >> (12 * k)) & 0xfffu; };
-    for (int h = 0; h < 2; ++h) {
-        const uint32_t c = e <= E ? cnt[e] : 0u;
-        const uint32_t nt0 = (c + trs[h] - 1) / trs[h];
-        const uint32_t nt = nt0 > 1 ? (nt0 + 1) & ~1u : nt0;
-        const uint32_t cls = nt > 1 ? 0u : 5u - min((c + 15) / 16, 4u);
-        const unsigned long long packed = (unsigned long long)nt << (12 * cls);
-        unsigned long long incl = packed;
-        for (int d = 1; d < 64; d <<= 1) {
-            const unsigned long long o = __shfl_up(incl, d, 64);
-            if ((int)lane >= d) incl += o;
-        }
-        __syncthreads();  // the previous list's wsum reads are done
-        if (lane == 63) wsum[wv] = incl;
-        __syncthreads();
-        unsigned long long off = incl - packed, all = 0;
-        for (uint32_t k = 0; k < wv; ++k) off += wsum[k];
-        for (uint32_t k = 0; k < PG_WG / 64; ++k) all += wsum[k];
-        uint32_t start = field(off, cls), total = 0;
-        for (uint32_t k = 0; k < 5; ++k) {
-            if (k < cls) start += field(all, k);
-            total += field(all, k);
-        }
-        uint2* tdst = tinfo + (dst - tiles);
-        for (uint32_t q = 0; q < nt; ++q) {
-            dst[start + q] = e << 16 | q;
-            tdst[start + q] = make_uint2(offs[e], cnt[e]);
-        }
-        if (tau == PG_WG - 1) ntiles[h] = total;
-        // bound of the first list, as pf_tile_bound computes it
-        const uint32_t n = (T * topk + tr - 1) / tr + E + (T + tr - 1) / tr + 1 + (E + 1);
-        dst = tiles + ((n + 15) & ~15u);
+    const uint32_t c = e <= E ? cnt[e] : 0u;
+    const uint32_t nt0 = (c + tr - 1) / tr;
+    const uint32_t nt = nt0 > 1 ? (nt0 + 1) & ~1u : nt0;
+    const uint32_t cls = nt > 1 ? 0u : 5u - min((c + 15) / 16, 4u);
+    const unsigned long long packed = (unsigned long long)nt << (12 * cls);
+    unsigned long long incl = packed;
+    for (int d = 1; d < 64; d <<= 1) {
+        const unsigned long long o = __shfl_up(incl, d, 64);
+        if ((int)lane >= d) incl += o;
     }
+    if (lane == 63) wsum[wv] = incl;
+    __syncthreads();
+    unsigned long long off = incl - packed, all = 0;
+    for (uint32_t k = 0; k < wv; ++k) off += wsum[k];
+    for (uint32_t k = 0; k < PG_WG / 64; ++k) all += wsum[k];
+    uint32_t start = field(off, cls), total = 0;
+    for (uint32_t k = 0; k < 5; ++k) {
+        if (k < cls) start += field(all, k);
+        total += field(all, k);
+    }
+    for (uint32_t q = 0; q < nt; ++q) {
+        tiles[start + q] = e << 16 | q;
+        tinfo[start + q] = make_uint2(offs[e], cnt[e]);
+    }
+    if (tau == PG_WG - 1) *ntiles = total;
 }
 
 // out[t][n] = sum_r w[t][r] yd[t][r][n] + sigmoid(sg[t]) yd[t][k][n]
@@ -1875,6 +1923,17 @@ static bool pf_gemm_prepare(PfGemmArgs& a, int epi) {
 }
 
 
+// Rows of the expert GEMMs' tiles: 32 where the groups average at most 8
+// rows (three workgroups fit a CU and each stages half the rows; 333 rows
+// over 512 experts: gate/up 167 -> 155 us, down 98 -> 89), 64 above (512
+// rows: equal; 2048: 317 against 340, a weight word unpacked for half the
+// rows).  Q2's 32-row form spills.
+uint32_t pf_tile_rows(const PfGemmArgs& gu, const PfGemmArgs& dn, uint32_t T, uint32_t topk, uint32_t E) {
+    if ((uint64_t)T * topk > 8ull * E || gu.X.bits == 2) return 64;
+    PfGemmArgs a = gu, b = dn;
+    return pf_gemm_prepare(a, PE_SILU_MUL) && pf_gemm_prepare(b, PE_STORE) ? 32 : 64;
+}
+
 bool launch_pf_gemm_args(const PfGemmArgs& args, int epi, uint32_t grid_y, hipStream_t st) {
     if (args.K % 64 || !args.K) throw std::runtime_error("prefill GEMM needs K a multiple of 64");
     if (!grid_y) return true;
@@ -1887,6 +1946,8 @@ bool launch_pf_gemm_args(const PfGemmArgs& args, int epi, uint32_t grid_y, hipSt
         a.phi = nullptr;
     if (a.phi && epi == PE_HC_UP && sbl) a.phi = nullptr;
     const bool fused = !args.phi || a.phi;
+    if (a.tinfo && a.trows != 64 && (a.trows != 32 || !sbl || a.ksplit > 1 || (a.X.base && a.X.bits == 2)))
+        throw std::runtime_error("grouped tiles of 64 rows, or of 32 with staged scales and 4- or 3-bit records");
     const uint32_t ksplit = std::max<uint32_t>(1, a.ksplit);
     if ((a.K / 64) % ksplit || (ksplit > 1 && epi != PE_STORE))
         throw std::runtime_error("split K needs whole groups per chunk and a plain store");
@@ -1909,6 +1970,19 @@ bool launch_pf_gemm_args(const PfGemmArgs& args, int epi, uint32_t grid_y, hipSt
         if (sbl) k_pf_gemm<NM, E, true><<<dim3(GX, grid_y, ksplit), PF_WG, 0, st>>>(a); \
         else k_pf_gemm<NM, E, false><<<dim3(GX, grid_y, ksplit), PF_WG, 0, st>>>(a);    \
     } while (0)
+    // Few rows: a launch of 64-row tiles that leaves CUs without a workgroup
+    // takes 32-row tiles, twice the workgroups with little over half the
+    // work each (a group's 73 unpack instructions are not shared by the
+    // halves; matrix and vector instructions of a SIMD hardly overlap, so a
+    // lone workgroup's step is their sum).  70 rows, 12288 outputs: 43 -> 28
+    // us; 256 rows (384 workgroups): 46 either way.
+    if (sbl && epi == PE_STORE && !a.tinfo) {
+        const uint32_t gx = (a.N + 255) / 256, gy = (a.M + 31) / 32;
+        if (gx * gy * ksplit <= PF_CUS || (a.K / 64 / ksplit <= 8 && gx * gy * ksplit <= 3 * PF_CUS)) {
+            k_pf_gemm<1, PE_STORE, true, 4, 2><<<dim3(gx, gy, ksplit), PF_WG, 0, st>>>(a);
+            return fused;
+        }
+    }
     const uint32_t xbits = a.X.base ? a.X.bits : 4;
     if (xbits != 4) {
         // grouped expert GEMMs over Q3 / Q2 records (scales staged where
@@ -1921,12 +1995,25 @@ bool launch_pf_gemm_args(const PfGemmArgs& args, int epi, uint32_t grid_y, hipSt
         if (epi == PE_STORE) k_pf_gemm<1, PE_STORE, S, B><<<grid, PF_WG, 0, st>>>(a);     \
         else k_pf_gemm<2, PE_SILU_MUL, S, B><<<grid, PF_WG, 0, st>>>(a);                  \
     } while (0)
+#define PF_LB2(B)                                                                         \
+    do {                                                                                  \
+        if (epi == PE_STORE) k_pf_gemm<1, PE_STORE, true, B, 2><<<grid, PF_WG, 0, st>>>(a); \
+        else k_pf_gemm<2, PE_SILU_MUL, true, B, 2><<<grid, PF_WG, 0, st>>>(a);            \
+    } while (0)
+        if (a.trows == 32 && xbits == 3) PF_LB2(3);
+        else
         if (xbits == 3 && sbl) PF_LB(3, true);
         else if (xbits == 3) PF_LB(3, false);
         else if (xbits == 2 && sbl) PF_LB(2, true);
         else if (xbits == 2) PF_LB(2, false);
         else throw std::runtime_error("expert records of 4, 3 or 2 bits");
 #undef PF_LB
+#undef PF_LB2
+        return fused;
+    }
+    if (a.tinfo && a.trows == 32) {
+        if (epi == PE_STORE) k_pf_gemm<1, PE_STORE, true, 4, 2><<<dim3((a.N + 255) / 256, grid_y), PF_WG, 0, st>>>(a);
+        else k_pf_gemm<2, PE_SILU_MUL, true, 4, 2><<<dim3((a.N + 127) / 128, grid_y), PF_WG, 0, st>>>(a);
         return fused;
     }
     switch (epi) {
@@ -1936,6 +2023,27 @@ bool launch_pf_gemm_args(const PfGemmArgs& args, int epi, uint32_t grid_y, hipSt
     }
 #undef PF_GEMM
     return fused;
+}
+
+void launch_pf_sum_parts(const PfGemmArgs& a, const float* part, uint32_t nsplit, uint32_t T, hipStream_t st) {
+    bool v4 = a.N % 4 == 0 && (uintptr_t)part % 16 == 0 && nsplit >= 1 && nsplit <= 4;
+    for (uint32_t q = 0; q < a.nseg; ++q)
+        v4 = v4 && (uintptr_t)a.seg[q].y % 16 == 0 && a.seg[q].ldy % 4 == 0 && a.seg[q].n0 % 4 == 0;
+    if (!v4) throw std::runtime_error("partial sums need 16-byte aligned segments of up to four chunks");
+    if (T) k_pf_sum_parts<<<dim3((a.N / 4 + CHK_WG - 1) / CHK_WG, T), CHK_WG, 0, st>>>(a, part, nsplit, T);
+}
+
+// K chunks of a GEMM whose consumer sums partials: the most, up to `most`,
+// that keep whole 8-group scale blocks and at most per_cu workgroups (of 64
+// rows) per CU.  [down; inject] of 8192 inputs, a chunk per stream: 43 us at
+// any T up to 1024; in up to 16 chunks 13 us at 256 rows, 20 at 512, 28 at
+// 1024 (2048 rows fill the CUs with a chunk per stream).  Out-projection
+// (4096 inputs): 43 -> 13 us at 128 rows, 21 at 256, 29 at 512.
+uint32_t pf_ksplit(uint32_t N, uint32_t K, uint32_t T, uint32_t least, uint32_t most, uint32_t per_cu) {
+    const uint32_t G = K / 64, wg = (N + 255) / 256 * ((T + 63) / 64);
+    uint32_t ks = least;
+    while (2 * ks <= most && G % (2 * ks) == 0 && G / (2 * ks) % 8 == 0 && wg * 2 * ks <= per_cu * PF_CUS) ks *= 2;
+    return ks;
 }
 
 void launch_pf_gemm(const Q4Mat& w, const uint4* xhi, const uint4* xlo, const float* xs, float* y, uint32_t T,
@@ -2014,11 +2122,11 @@ void launch_pf_group(uint32_t* gcnt, uint32_t T, uint32_t topk, uint32_t E, uint
                      uint32_t tr, bool shared, hipStream_t st) {
     if (E + 1 > PG_WG) throw std::runtime_error("prefill grouping supports at most 1023 experts");
     if (T > cap || (uint64_t)T * (topk + 1) >= (1u << 22)) throw std::runtime_error("prefill grouping: too many entries");
-    if (tr != 48 && tr != 64) throw std::runtime_error("prefill grouping: tiles of 48 or 64 rows");
-    if (pf_tile_bound(T, topk, E, tr) >= 0x1000u || pf_tile_bound(T, topk, E, 64) >= 0x1000u)
+    if (tr != 32 && tr != 64) throw std::runtime_error("prefill grouping: tiles of 32 or 64 rows");
+    if (pf_tile_bound(T, topk, E, tr) >= 0x1000u)
         throw std::runtime_error("prefill grouping: too many tiles");
     k_pf_group<<<1, PG_WG, 0, st>>>(gcnt, T, E, cap, count, tiles, ntiles, tinfo, goff,
-                                    reinterpret_cast<unsigned long long*>(act), layer, tr, topk, shared ? 1u : 0u);
+                                    reinterpret_cast<unsigned long long*>(act), layer, tr, shared ? 1u : 0u);
 }
 
 // Tiles of a grouped GEMM: every group's rows in tr-row tiles, one more

@@ -1,0 +1,44 @@
+"""The prefill GEMMs' forms for few rows: 32-row tiles, K chunks of the
+hyper-connection, input and out projections (their partials summed by the
+next pass), expert tiles of 32 rows.  One layer of the 80B shape at row
+counts around the tiles and around each rule's bound, with room for the
+partials and without, against the row path."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from cherenkov_amd import presets
+from cherenkov_amd.engine import Engine
+from tests.gpu_util import assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bits,interval", [(4, 4), (4, 1), (3, 4), (2, 4)])
+def test_few_rows_match_row_path(have_gpu, bits, interval):
+    cfg = presets.qwen3next_80b_shape(layers=1, mtp=0)
+    cfg.full_attention_interval = interval
+    toks = np.random.default_rng(bits * 10 + interval).integers(0, cfg.vocab_size, size=450).tolist()
+    rows = [1, 15, 16, 17, 33, 65, 128, 129, 161, 300] + ([410, 450] if bits == 4 and interval == 4 else [])
+    b = Engine(cfg, experts=bits, drafts=0, max_t=512)
+    ref = {}
+    try:
+        for i, t in enumerate(toks[:max(rows)]):
+            b.step(t)
+            if i + 1 in rows:
+                ref[i + 1] = b.logits()
+    finally:
+        b.close()
+    for max_t in (2048, 512):  # partials of many rows fit / do not fit
+        a = Engine(cfg, experts=bits, drafts=0, max_t=max_t)
+        try:
+            for n in rows:
+                a.reset()
+                a.prefill_chunk(toks[:n])
+                # one layer: only the last row's own routing matters; f32-grade
+                # sums in another order
+                assert_close(a.logits(), ref[n], f"{bits} bits, {n} rows, max_t {max_t}", abs_frac=1e-3, min_cos=0.99999)
+        finally:
+            a.close()
