@@ -173,12 +173,13 @@ struct PfBufs {
     // the normed trunk streams, fc_e / fc_h outputs and the head's residual
     uint32_t* mtp_tok;
     float *mtp_en, *mtp_hn, *mtp_fe, *mtp_fh, *mtp_hyper;
-    // the flash attention plan (pf_flash_split) for the chunk's rows,
+    // the flash attention plan (pf_flash_plan, pf_flash_split) for the chunk's rows,
     // uploaded for the (rows, first position) key it was made for (its
     // partials take yd, free between an attention block's
     // hyper-connection read and its out-projection)
     uint4 *fa_seg, *fa_merge;
     uint64_t fa_key = ~0ull;
+    bool first = false;  // the chunk starts at position 0
     uint32_t fa_W = 0, fa_nslots = 0, fa_nmerge = 0;
     // QSA past the budget: every row's index queries; block scores of
     // qsa_rows rows at a time
@@ -1508,6 +1509,11 @@ struct ChkEngine {
         const uint32_t g = D.nh / D.nkv;
         return C * (D.topk + 1) * D.H / ((uint64_t)D.nkv * pf_flash_rows(g) * g * (2 + D.hd));
     }
+    // yd: the expert down outputs, or a first chunk's partials of two 16-row
+    // blocks per workgroup
+    uint64_t yd_floats(uint64_t C) const {
+        return std::max<uint64_t>(C * (D.topk + 1) * D.H, 2 * std::min<uint64_t>((C + 15) / 16, fa_wmax(C)) * 16 * D.nh * (2 + D.hd));
+    }
     uint32_t pf_dense_rows(uint32_t T, uint32_t pos0) const;
     PfFlashLaunch pf_flash_launch(uint32_t T, uint32_t pos0);
     uint32_t pf_qsa_rows(uint64_t C) const;
@@ -1747,7 +1753,7 @@ uint64_t ChkEngine::prefill_scratch_bytes(uint64_t C, bool all_logits) const {
     b += C * (PF_ROUTER_CHUNKS * D.E + 1 + 2ull * D.topk) * f + (D.E + 1ull) * C * 4 +
          (PF_GCNT_STRIDE + 1ull) * (D.E + 1) * 4;
     b += (uint64_t)(pf_tile_bound((uint32_t)C, D.topk, D.E, 32)) * 12 +
-         C * slots * (D.I + D.H) * f + C * slots * 4 + (D.E + 1) * 4;
+         (C * slots * D.I + yd_floats(C)) * f + C * slots * 4 + (D.E + 1) * 4;
     if (D.SI != D.I) b += C * D.SI * f;
     if (dc_supported(D.nk, D.nv, D.dk, D.dv)) b += dc_work_floats((uint32_t)C, D.nv, D.dv) * f;
     if (all_logits) b += C * D.V * f;
@@ -1876,7 +1882,7 @@ void ChkEngine::pf_alloc() {
     pf.ntiles = pfalloc<uint32_t>(1);
     pf.act = pfalloc<float>(C * slots * D.I);
     pf.act_sh = D.SI != D.I ? pfalloc<float>(C * D.SI) : nullptr;
-    pf.yd = pfalloc<float>(C * slots * D.H);
+    pf.yd = pfalloc<float>(yd_floats(C));
     pf.dcw = dc_supported(D.nk, D.nv, D.dk, D.dv) ? pfalloc<float>(dc_work_floats((uint32_t)C, D.nv, D.dv)) : nullptr;
     if (D.qsa) {
         pf.qsa_rows = pf_qsa_rows(C);
@@ -1926,7 +1932,7 @@ void ChkEngine::pf_hc_read(const HcDev& w, float* inj, uint32_t T, bool for_moe)
     g.N = N;
     g.K = D.hh;
     g.M = T;
-    g.ksplit = pf_ksplit(N, D.hh, T, D.hc, (uint32_t)std::min<uint64_t>(16, std::max(act_fit, own_fit)));
+    g.ksplit = pf.first ? D.hc : pf_ksplit(N, D.hh, T, D.hc, (uint32_t)std::min<uint64_t>(16, std::max(act_fit, own_fit)));
     g.zstride = (uint64_t)T * N;
     g.xhi = pf.hi;
     g.xlo = pf.lo;
@@ -1995,7 +2001,7 @@ void ChkEngine::pf_out_proj(const Q4Mat& m, uint32_t K, uint32_t T) {
     o.N = D.H;
     o.K = K;
     o.M = T;
-    o.ksplit = G % 2 == 0 && (G / 2) % 8 == 0 ? pf_ksplit(D.H, K, T, 2, std::min<uint32_t>(8, D.topk + 1)) : 1;
+    o.ksplit = G % 2 == 0 && (G / 2) % 8 == 0 ? pf_ksplit(D.H, K, T, 2, pf.first ? 2 : std::min<uint32_t>(8, D.topk + 1)) : 1;
     o.zstride = (uint64_t)pf.cap * D.H;
     o.xhi = pf.hi;
     o.xlo = pf.lo;
@@ -2011,7 +2017,7 @@ void ChkEngine::pf_out_proj(const Q4Mat& m, uint32_t K, uint32_t T) {
 void ChkEngine::pf_in_proj(const PfGemmArgs& g, uint32_t T) {
     const uint64_t fit = (uint64_t)pf.cap * (D.topk + 1) * D.H / ((uint64_t)T * g.N);
     const uint32_t ks = pf_ksplit(g.N, g.K, T, 1, (uint32_t)std::min<uint64_t>(4, fit), 2);
-    if (ks < 4 || g.N % 4) {
+    if (pf.first || ks < 4 || g.N % 4) {
         launch_pf_gemm_args(g, PE_STORE, (T + 63) / 64, st);
         return;
     }
@@ -2186,9 +2192,12 @@ uint32_t ChkEngine::pf_dense_rows(uint32_t T, uint32_t pos0) const {
 PfFlashLaunch ChkEngine::pf_flash_launch(uint32_t T, uint32_t pos0) {
     const uint64_t key = (uint64_t)T << 32 | pos0;
     if (key != pf.fa_key) {
-        const PfFlashPlan p = pf_flash_split(T, pos0, fa_wmax(pf.cap), pf_flash_rows(D.nh / D.nkv), fa_slots(pf.cap));
+        const bool first = pf.first && pf_dense_rows(T, pos0) == T;
+        const PfFlashPlan p = first ? pf_flash_plan(T, 0, std::max<uint32_t>(1, ncu / D.nkv))
+                                    : pf_flash_split(T, pos0, fa_wmax(pf.cap), pf_flash_rows(D.nh / D.nkv), fa_slots(pf.cap));
         const uint64_t n = fa_entries(pf.cap);
-        if (p.seg.size() > n * FA_MAXSEG || p.merge.size() > n || p.nslots > fa_slots(pf.cap))
+        const uint64_t slots = first ? yd_floats(pf.cap) / (16ull * D.nh * (2 + D.hd)) : fa_slots(pf.cap);
+        if (p.seg.size() > n * FA_MAXSEG || p.merge.size() > n || p.nslots > slots)
             throw std::runtime_error("flash attention plan exceeds its buffers");
         HIPCHK(hipStreamSynchronize(st));
         HIPCHK(hipMemcpy(pf.fa_seg, p.seg.data(), p.seg.size() * sizeof(uint4), hipMemcpyHostToDevice));
@@ -2324,6 +2333,9 @@ void ChkEngine::prefill_gemm(const uint32_t* toks, uint32_t n, uint32_t next_aft
         pf.pend = nullptr;  // (an earlier failed chunk may have left one)
         pf.moe_pend = nullptr;
         HIPCHK(hipMemsetAsync(pf.gcnt, 0, (D.E + 1) * PF_GCNT_STRIDE * 4, st));  // (and its expert counts)
+        // a prompt's first chunk keeps the K chunk counts and the attention
+        // form of its sums (k_pf_flash_first)
+        pf.first = pos0 == 0;
         // the chunk's flash plan, while the stream is idle
         pf_flash_launch(T, pos0);
         launch_pf_embed(pf.tokens, embed, pf.hyper, D.H, D.hc, T, st);

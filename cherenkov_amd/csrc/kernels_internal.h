@@ -477,15 +477,16 @@ struct PfFlashPlan {
 };
 // rows of a row block: a workgroup's eight waves serve `g` query heads
 constexpr uint32_t pf_flash_rows(uint32_t g) { return g >= 8 ? 16u : 16u * (8u / g); }
+// (a prompt's first chunk, see pf_flash_first, takes this plan over 16-row blocks)
 PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows = 16, bool whole_only = false);
-// the plan the engine takes: pf_flash_plan, or where the chunk has fewer row
-// blocks than max_wg, its steps over more workgroups than row blocks; at
-// most max_slots partial slots
+// the plan behind a context or past the QSA budget: pf_flash_plan, or where
+// the chunk has fewer row blocks than max_wg, its steps over more workgroups
+// than row blocks; at most max_slots partial slots
 PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows = 16, uint64_t max_slots = ~0ull);
 struct PfFlashLaunch {         // a plan uploaded to the device
     const uint4* seg;
     const uint4* merge;
-    float* part;               // [nkv][nslots][rows][nh / nkv][2 + hd]
+    float* part;               // [nkv][nslots][rows][nh / nkv][2 + hd], rows 16 or pf_flash_rows
     uint32_t W, nslots, nmerge;
 };
 // QSA: the rows' block selections (vmask null: every row attends densely)
@@ -493,6 +494,8 @@ struct PfFlashSel {
     const uint32_t* vmask = nullptr;  // [T][mask_words]
     uint32_t mask_words = 0, ratio = 1, kblk = 0;
 };
+// whether a chunk's attention runs in k_pf_flash_first's form
+constexpr bool pf_flash_first(uint32_t pos0, const void* vmask) { return pos0 == 0 && !vmask; }
 void launch_pf_flash(const float* q_ready, const float* q_raw, const KvDev& kv, float* out, uint32_t T, uint32_t pos0,
                      uint32_t nh, uint32_t nkv, uint32_t hd, float scale, const PfFlashLaunch& plan, hipStream_t st,
                      const PfFlashSel& sel = PfFlashSel{});

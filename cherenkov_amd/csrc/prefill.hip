@@ -2038,7 +2038,8 @@ void launch_pf_sum_parts(const PfGemmArgs& a, const float* part, uint32_t nsplit
 // rows) per CU.  [down; inject] of 8192 inputs, a chunk per stream: 43 us at
 // any T up to 1024; in up to 16 chunks 13 us at 256 rows, 20 at 512, 28 at
 // 1024 (2048 rows fill the CUs with a chunk per stream).  Out-projection
-// (4096 inputs): 43 -> 13 us at 128 rows, 21 at 256, 29 at 512.
+// (4096 inputs): 43 -> 13 us at 128 rows, 21 at 256, 29 at 512.  The engine
+// asks for more than `least` behind a context only (see k_pf_flash_first).
 uint32_t pf_ksplit(uint32_t N, uint32_t K, uint32_t T, uint32_t least, uint32_t most, uint32_t per_cu) {
     const uint32_t G = K / 64, wg = (N + 255) / 256 * ((T + 63) / 64);
     uint32_t ks = least;
@@ -2220,6 +2221,7 @@ struct PfFlashArgs {
     float* out;            // [T][nh * hd]
     uint32_t T, pos0, nh, nkv;
     float scale2;          // the softmax scale times log2 e
+    float scale;
     const uint4* seg;      // [W][FA_MAXSEG] the plan's segments (pf_flash_plan)
     float* part;           // [nkv][nslots][rows][G][2 + hd] partials of split row blocks
     uint32_t nslots;
@@ -2642,6 +2644,301 @@ __global__ void __launch_bounds__(256) k_pf_flash_join(PfFlashArgs a, const uint
         op[j] = fd{O[2 * j] * inv * sigmoidf_(gate[j].x), O[2 * j + 1] * inv * sigmoidf_(gate[j].y)};
 }
 
+// A prompt's first chunk, every row within the budget: the same work in
+// 16-row blocks, a wave per query head of the kv head.  Within a segment,
+// wave w serves the kv head's query head w (the group's waves share every
+// staged K/V tile).  Per 32-token tile the workgroup dequantises K and V
+// (int8 x fp16 scale, exact in f32) into LDS as fp16 hi + lo planes (V
+// transposed), then each wave runs S = Q K^T and O += P V in three passes
+// (hi.hi + hi.lo + lo.hi) and an online softmax in f32.
+// 2048 rows of 16 heads of 256 over 2: 180 + 19 us (k_pf_flash 156 + 14,
+// 0.3 ms of a 48-layer prompt's 65).  It stays for its sums: a prompt's
+// roundings choose the cache codes and near-tied experts that its answer
+// goes on with, so a prompt answers as before (48 layers behind 2048
+// tokens: logits 3.5e-3 apart between the two forms, each within 1.8e-6 of
+// 64 bits over one layer).
+template <int HD, int G>
+__global__ void __launch_bounds__(64 * G) k_pf_flash_first(PfFlashArgs a) {
+    constexpr int KS = HD / 32;          // dim steps of 32
+    constexpr int DT = HD / 16;          // 16-dim output tiles
+    constexpr int KP = HD + 8;           // padded K row (halves)
+    constexpr int VP = FA_TOK + 8;       // padded V^T row (halves)
+    constexpr int PP = FA_TOK + 8;       // padded P row (halves)
+    __shared__ __align__(16) _Float16 kh[FA_TOK][KP], kl[FA_TOK][KP];
+    __shared__ __align__(16) _Float16 vh[HD][VP], vl[HD][VP];
+    __shared__ __align__(16) _Float16 ph[G][FA_ROWS][PP], pl[G][FA_ROWS][PP];
+    constexpr uint32_t nthr = 64 * G;
+    constexpr int IPT = (FA_TOK * HD / 16 + nthr - 1) / nthr;  // staging items per thread
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = wave_id();
+    const uint32_t col = lane & 15, kq = lane >> 4;
+    const uint32_t hk = blockIdx.y, h = hk * G + w;
+    const uint32_t kv_row = a.nkv * HD, last_tok = a.pos0 + a.T - 1;
+    const uint4* segs = a.seg + (size_t)blockIdx.x * FA_MAXSEG;
+    for (uint32_t sgi = 0; sgi < FA_MAXSEG; ++sgi) {
+    const uint4 sg = segs[sgi];  // (row block, first tile, end tile, slot or ~0: the whole block)
+    if (sg.x == ~0u) break;
+    if (sgi) __syncthreads();  // every wave is done with the previous segment's tiles
+    const uint32_t rb = sg.x, ta = sg.y, tb = sg.z;
+    const uint32_t r0 = rb * FA_ROWS;
+    // this wave's queries as A operands
+    h8 qh[KS], ql[KS];
+    {
+        const uint32_t r = min(r0 + col, a.T - 1);
+        const float* qp = a.q_ready + ((size_t)r * a.nh + h) * HD;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const float4 v0 = *reinterpret_cast<const float4*>(qp + s * 32 + kq * 8);
+            const float4 v1 = *reinterpret_cast<const float4*>(qp + s * 32 + kq * 8 + 4);
+            const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+            qh[s] = split_hi(v, ql[s]);
+        }
+    }
+    // positions of the 4 rows this lane holds in D layout (rows past T
+    // repeat the last row; they are never written)
+    uint32_t qpos[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) qpos[i] = a.pos0 + min(r0 + kq * 4 + i, a.T - 1);
+    f4 o[DT];
+#pragma unroll
+    for (int d = 0; d < DT; ++d) o[d] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    float m[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        m[i] = -INFINITY;
+        l[i] = 0.0f;
+    }
+    // Staging: K as (token tid % 32, 16 dims), V as (token pair tid % 16,
+    // 8 dims) so that the transposed V writes are whole dwords in
+    // consecutive banks; a tile's raw bytes are loaded one tile ahead.
+    uint4 kraw[IPT];
+    uint2 vraw[IPT][2];
+    uint16_t ksc[IPT], vsc[IPT][2];
+    auto load_raw = [&](uint32_t t0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < IPT; ++r) {
+            const uint32_t i = tid + r * nthr;
+            kraw[r] = make_uint4(0, 0, 0, 0);
+            vraw[r][0] = vraw[r][1] = make_uint2(0, 0);
+            ksc[r] = vsc[r][0] = vsc[r][1] = 0;
+            if (i >= (uint32_t)(FA_TOK * HD / 16)) continue;
+            const uint32_t kt = t0 + i % FA_TOK, kd = (i / FA_TOK) * 16;
+            if (kt <= last_tok) {
+                kraw[r] = *reinterpret_cast<const uint4*>(a.kv.k + (size_t)kt * kv_row + hk * HD + kd);
+                ksc[r] = a.kv.ks[(size_t)kt * (kv_row / 32) + (hk * HD + kd) / 32];
+            }
+            const uint32_t vt = t0 + 2 * (i % (FA_TOK / 2)), vd = (i / (FA_TOK / 2)) * 8;
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                if (vt + e <= last_tok) {
+                    vraw[r][e] = *reinterpret_cast<const uint2*>(a.kv.v + (size_t)(vt + e) * kv_row + hk * HD + vd);
+                    vsc[r][e] = a.kv.vs[(size_t)(vt + e) * (kv_row / 32) + (hk * HD + vd) / 32];
+                }
+        }
+    };
+    auto store_tile = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < IPT; ++r) {
+            const uint32_t i = tid + r * nthr;
+            if (i >= (uint32_t)(FA_TOK * HD / 16)) continue;
+            const uint32_t kt = i % FA_TOK, kd = (i / FA_TOK) * 16;
+            const float kscale = __half2float(__ushort_as_half(ksc[r]));
+            const uint32_t kwv[4] = {kraw[r].x, kraw[r].y, kraw[r].z, kraw[r].w};
+#pragma unroll
+            for (int hlf = 0; hlf < 2; ++hlf) {
+                float kv8[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    kv8[j] = (float)(int8_t)(kwv[hlf * 2 + j / 4] >> (8 * (j % 4))) * kscale;
+                h8 lo8;
+                const h8 hi8 = split_hi(kv8, lo8);
+                *reinterpret_cast<h8*>(&kh[kt][kd + hlf * 8]) = hi8;
+                *reinterpret_cast<h8*>(&kl[kt][kd + hlf * 8]) = lo8;
+            }
+            const uint32_t vt = 2 * (i % (FA_TOK / 2)), vd = (i / (FA_TOK / 2)) * 8;
+            const float vs0 = __half2float(__ushort_as_half(vsc[r][0])), vs1 = __half2float(__ushort_as_half(vsc[r][1]));
+            const uint32_t v0[2] = {vraw[r][0].x, vraw[r][0].y}, v1[2] = {vraw[r][1].x, vraw[r][1].y};
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float x0 = (float)(int8_t)(v0[j / 4] >> (8 * (j % 4))) * vs0;
+                const float x1 = (float)(int8_t)(v1[j / 4] >> (8 * (j % 4))) * vs1;
+                const _Float16 h0 = (_Float16)x0, h1 = (_Float16)x1;
+                typedef _Float16 hh2 __attribute__((ext_vector_type(2)));
+                *reinterpret_cast<hh2*>(&vh[vd + j][vt]) = hh2{h0, h1};
+                *reinterpret_cast<hh2*>(&vl[vd + j][vt]) = hh2{(_Float16)(x0 - (float)h0), (_Float16)(x1 - (float)h1)};
+            }
+        }
+    };
+    load_raw(ta * FA_TOK);
+    store_tile();
+    __syncthreads();
+    for (uint32_t tile = ta; tile < tb; ++tile) {
+        const uint32_t t0 = tile * FA_TOK;
+        if (tile + 1 < tb) load_raw(t0 + FA_TOK);
+        // ---- S = Q K^T for 2 token tiles
+        f4 s[2];
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            s[tt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const h8 bh = *reinterpret_cast<const h8*>(&kh[tt * 16 + col][ks * 32 + kq * 8]);
+                const h8 bl = *reinterpret_cast<const h8*>(&kl[tt * 16 + col][ks * 32 + kq * 8]);
+                s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ql[ks], bh, s[tt], 0, 0, 0);
+                s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[ks], bl, s[tt], 0, 0, 0);
+                s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[ks], bh, s[tt], 0, 0, 0);
+            }
+        }
+        // ---- online softmax over the tile (rows kq*4 + i, tokens col, 16 + col)
+        float p[2][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float mx = -INFINITY;
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+                const uint32_t t = t0 + tt * 16 + col;
+                const float v = t <= qpos[i] ? s[tt][i] * a.scale : -INFINITY;
+                p[tt][i] = v;
+                mx = fmaxf(mx, v);
+            }
+            mx = group_max<16>(mx);
+            const float mn = fmaxf(m[i], mx);
+            const float corr = m[i] == -INFINITY ? 0.0f : expf(m[i] - mn);
+            float rs = 0.0f;
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+                const float e = p[tt][i] == -INFINITY ? 0.0f : expf(p[tt][i] - mn);
+                p[tt][i] = e;
+                rs += e;
+            }
+            rs = group_sum<16>(rs);
+            l[i] = l[i] * corr + rs;
+            m[i] = mn;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) o[d][i] *= corr;
+        }
+        // ---- P to this wave's LDS rows (hi, lo), read back as A operands:
+        // LDS instructions of one wave complete in order, so only the
+        // compiler has to be kept from reordering them
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const _Float16 hi = (_Float16)p[tt][i];
+                ph[w][kq * 4 + i][tt * 16 + col] = hi;
+                pl[w][kq * 4 + i][tt * 16 + col] = (_Float16)(p[tt][i] - (float)hi);
+            }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const h8 pah = *reinterpret_cast<const h8*>(&ph[w][col][kq * 8]);
+        const h8 pal = *reinterpret_cast<const h8*>(&pl[w][col][kq * 8]);
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+            const h8 bh = *reinterpret_cast<const h8*>(&vh[d * 16 + col][kq * 8]);
+            const h8 bl = *reinterpret_cast<const h8*>(&vl[d * 16 + col][kq * 8]);
+            o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pal, bh, o[d], 0, 0, 0);
+            o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pah, bl, o[d], 0, 0, 0);
+            o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pah, bh, o[d], 0, 0, 0);
+        }
+        if (tile + 1 < tb) {
+            __syncthreads();  // every wave is done with this tile's K and V
+            store_tile();
+            __syncthreads();
+        }
+    }
+    if (sg.w == ~0u) {
+        // ---- o / l times the per-dim sigmoid gate (cpu.rs:629-633)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t r = r0 + kq * 4 + i;
+            if (r >= a.T) continue;
+            const float inv = 1.0f / l[i];
+            const float* gp = a.q_raw + ((size_t)r * a.nh + h) * 2 * HD + HD;
+            float* op = a.out + (size_t)r * a.nh * HD + (size_t)h * HD;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                const uint32_t dd = d * 16 + col;
+                op[dd] = o[d][i] * inv * sigmoidf_(gp[dd]);
+            }
+        }
+    } else {
+        // ---- a piece of a split row block: (m, l, unnormalised o) per row
+        float* pp = a.part + ((size_t)hk * a.nslots + sg.w) * FA_ROWS * G * (2 + HD);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float* q = pp + ((size_t)(kq * 4 + i) * G + w) * (2 + HD);
+            if (col == 0) {
+                q[0] = m[i];
+                q[1] = l[i];
+            }
+#pragma unroll
+            for (int d = 0; d < DT; ++d) q[2 + d * 16 + col] = o[d][i];
+        }
+    }
+    }
+}
+
+// Joins the pieces of k_pf_flash_first's split row blocks: per row, head and
+// dim, o = sum_k o_k e^(m_k - M) / sum_k l_k e^(m_k - M) with M = max_k m_k
+// (a piece whose tokens a row cannot see holds m = -inf, l = 0), times the
+// sigmoid gate.  Workgroup (entry, row) of kv head blockIdx.z; thread d
+// takes dims d, d + 256 of every head, all loads issued before the sums.
+template <int G, int HD>
+__global__ void __launch_bounds__(256) k_pf_first_merge(PfFlashArgs a, const uint4* __restrict__ merge) {
+    constexpr int DPT = (HD + CHK_WG - 1) / CHK_WG;
+    const uint4 me = merge[blockIdx.x];  // (row block, first slot, pieces, 0)
+    const uint32_t row = blockIdx.y, hk = blockIdx.z, r = me.x * FA_ROWS + row, np = me.z;
+    if (r >= a.T) return;
+    const float* __restrict__ part = a.part;
+    const float* __restrict__ qraw = a.q_raw;
+    float* __restrict__ outp = a.out;
+    const size_t ps = (size_t)FA_ROWS * G * (2 + HD);  // floats per slot
+    const float* p0 = part + ((size_t)hk * a.nslots + me.y) * ps + (size_t)row * G * (2 + HD);
+    float mk[G][FA_MAXP], lk[G][FA_MAXP], ok[G][FA_MAXP][DPT], gate[G][DPT];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const float* q = p0 + (size_t)g * (2 + HD);
+#pragma unroll
+        for (int k = 0; k < FA_MAXP; ++k) {
+            const bool on = (uint32_t)k < np;
+            mk[g][k] = on ? q[k * ps] : -INFINITY;
+            lk[g][k] = on ? q[k * ps + 1] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < DPT; ++j) {
+                const uint32_t d = threadIdx.x + j * CHK_WG;
+                ok[g][k][j] = on && d < (uint32_t)HD ? q[k * ps + 2 + d] : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < DPT; ++j) {
+            const uint32_t d = min(threadIdx.x + j * CHK_WG, (uint32_t)HD - 1);
+            gate[g][j] = qraw[((size_t)r * a.nh + hk * G + g) * 2 * HD + HD + d];
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        float M = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < FA_MAXP; ++k) M = fmaxf(M, mk[g][k]);
+        float e[FA_MAXP], L = 0.0f;
+#pragma unroll
+        for (int k = 0; k < FA_MAXP; ++k) {
+            e[k] = mk[g][k] == -INFINITY ? 0.0f : expf(mk[g][k] - M);
+            L += lk[g][k] * e[k];
+        }
+        const float inv = 1.0f / L;
+#pragma unroll
+        for (int j = 0; j < DPT; ++j) {
+            const uint32_t d = threadIdx.x + j * CHK_WG;
+            if (d >= (uint32_t)HD) continue;
+            float O = 0.0f;
+#pragma unroll
+            for (int k = 0; k < FA_MAXP; ++k) O += ok[g][k][j] * e[k];
+            outp[(size_t)r * a.nh * HD + (size_t)(hk * G + g) * HD + d] = O * inv * sigmoidf_(gate[g][j]);
+        }
+    }
+}
+
 // Deals every kv head's (row block, tile) steps to max_wg workgroups in
 // equal shares (see k_pf_flash); one whole row block per workgroup, heavy
 // ones first, where the blocks' work is within 15% of even or a share
@@ -2704,8 +3001,8 @@ PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t r
     return p;
 }
 
-// The plan of a chunk with fewer row blocks than workgroups (a short prompt
-// or message, mostly behind a long context): every kv head's steps, row
+// The plan of a chunk with fewer row blocks than workgroups (a message
+// behind a context): every kv head's steps, row
 // block after row block, cut into equal ranges over up to max_wg
 // workgroups of at least FA_MINSHARE tiles each, so a row block is split
 // over as many workgroups as its context fills.  One workgroup per row
@@ -2757,12 +3054,35 @@ void launch_pf_flash(const float* q_ready, const float* q_raw, const KvDev& kv, 
     if (!T) return;
     if (!plan.seg || !plan.W || (plan.nmerge && (!plan.merge || !plan.part)))
         throw std::runtime_error("flash prefill needs its plan");
-    PfFlashArgs a{q_ready, q_raw, kv, out, T, pos0, nh, nkv, scale * 1.44269504088896341f, plan.seg, plan.part, plan.nslots,
+    PfFlashArgs a{q_ready, q_raw, kv, out, T, pos0, nh, nkv, scale * 1.44269504088896341f, scale, plan.seg, plan.part, plan.nslots,
                   sel.vmask, sel.mask_words, sel.kblk, 1.0f / (float)sel.ratio};
     const dim3 grid(plan.W, nkv);
     const uint32_t g = nh / nkv;
     if (g != 1 && g != 2 && g != 4 && g != 8)
         throw std::runtime_error("flash prefill takes 1, 2, 4 or 8 query heads per kv head");
+    if (pf_flash_first(pos0, sel.vmask)) {
+        const dim3 mgrid(plan.nmerge, FA_ROWS, nkv);
+#define CHK_FA(HDV, GV)                                                                          \
+    {                                                                                            \
+        k_pf_flash_first<HDV, GV><<<grid, 64 * GV, 0, st>>>(a);                                  \
+        if (plan.nmerge) k_pf_first_merge<GV, HDV><<<mgrid, CHK_WG, 0, st>>>(a, plan.merge);     \
+        break;                                                                                   \
+    }
+        if (hd == 256) switch (g) {
+            case 1: CHK_FA(256, 1)
+            case 2: CHK_FA(256, 2)
+            case 4: CHK_FA(256, 4)
+            default: CHK_FA(256, 8)
+            }
+        else switch (g) {
+            case 1: CHK_FA(128, 1)
+            case 2: CHK_FA(128, 2)
+            case 4: CHK_FA(128, 4)
+            default: CHK_FA(128, 8)
+            }
+#undef CHK_FA
+        return;
+    }
 #define CHK_FA(HDV, SELV)                                                        \
     switch (g) {                                                                 \
     case 1: k_pf_flash<HDV, 1, SELV><<<grid, 512, 0, st>>>(a); break;            \

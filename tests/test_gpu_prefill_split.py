@@ -1,7 +1,8 @@
 """The prefill GEMMs' forms for few rows: 32-row tiles, K chunks of the
 hyper-connection, input and out projections (their partials summed by the
 next pass), expert tiles of 32 rows.  One layer of the 80B shape at row
-counts around the tiles and around each rule's bound, with room for the
+counts around the tiles and around each rule's bound, as a prompt's first
+chunk (which keeps its K chunks) and behind a context, with room for the
 partials and without, against the row path."""
 
 from __future__ import annotations
@@ -20,25 +21,27 @@ pytestmark = pytest.mark.gpu
 def test_few_rows_match_row_path(have_gpu, bits, interval):
     cfg = presets.qwen3next_80b_shape(layers=1, mtp=0)
     cfg.full_attention_interval = interval
-    toks = np.random.default_rng(bits * 10 + interval).integers(0, cfg.vocab_size, size=450).tolist()
+    toks = np.random.default_rng(bits * 10 + interval).integers(0, cfg.vocab_size, size=455).tolist()
     rows = [1, 15, 16, 17, 33, 65, 128, 129, 161, 300] + ([410, 450] if bits == 4 and interval == 4 else [])
     b = Engine(cfg, experts=bits, drafts=0, max_t=512)
     ref = {}
     try:
-        for i, t in enumerate(toks[:max(rows)]):
+        for i, t in enumerate(toks[:max(rows) + 5]):
             b.step(t)
-            if i + 1 in rows:
+            if i + 1 in rows or i - 4 in rows:
                 ref[i + 1] = b.logits()
     finally:
         b.close()
     for max_t in (2048, 512):  # partials of many rows fit / do not fit
         a = Engine(cfg, experts=bits, drafts=0, max_t=max_t)
         try:
-            for n in rows:
+            for n, ctx in [(n, ctx) for n in rows for ctx in (0, 5)]:
                 a.reset()
-                a.prefill_chunk(toks[:n])
+                if ctx:
+                    a.prefill_chunk(toks[:ctx])
+                a.prefill_chunk(toks[ctx:ctx + n])
                 # one layer: only the last row's own routing matters; f32-grade
                 # sums in another order
-                assert_close(a.logits(), ref[n], f"{bits} bits, {n} rows, max_t {max_t}", abs_frac=1e-3, min_cos=0.99999)
+                assert_close(a.logits(), ref[ctx + n], f"{bits} bits, {n} rows behind {ctx}, max_t {max_t}", abs_frac=1e-3, min_cos=0.99999)
         finally:
             a.close()
