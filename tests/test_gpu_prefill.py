@@ -43,6 +43,23 @@ def test_q4_gemm_matches_rowwise_oracle(have_gpu, out_dim, in_dim, T):
     assert_close(got, ref, f"gemm {out_dim}x{in_dim} T={T}", abs_frac=1e-4, min_cos=0.999999)
 
 
+@pytest.mark.parametrize("out_dim,in_dim,T", [(333, 512, 100), (1, 64, 1)])
+@pytest.mark.parametrize("words", [1, 2])
+def test_q4_gemm_codes_off_their_alignment(have_gpu, out_dim, in_dim, T, words):
+    """Codes on any word boundary: the same bits as aligned ones, read in place."""
+    rng = np.random.default_rng(out_dim + T)
+    w, s, b = rand_q4(rng, out_dim, in_dim)
+    shifted = np.concatenate([np.zeros(words, np.uint32), w.ravel()])
+    dw, dv, ds, db = to_dev(w), to_dev(shifted), to_dev(s), to_dev(b)
+    dx = to_dev(rng.normal(0, 1, (T, in_dim)).astype(np.float32))
+    got = []
+    for at in (dw.data_ptr(), dv.data_ptr() + 4 * words):
+        y = empty_dev((T, out_dim))
+        check(lib().chk_q4_gemm(at, ds.data_ptr(), db.data_ptr(), out_dim, in_dim, dx.data_ptr(), T, y.data_ptr(), None))
+        got.append(to_host(y))
+    assert np.array_equal(got[0], got[1])
+
+
 def row_prefill(eng, prompt):
     out = None
     for t in prompt:
