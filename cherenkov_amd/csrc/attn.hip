@@ -488,7 +488,15 @@ CHK_DEV float h2f(uint16_t h) { return __half2float(__ushort_as_half(h)); }
 // Scores: 4 threads per token, each a quarter of the head dims (HD / 4,
 // i.e. HD / 128 q8 blocks of 32).  P.V: lanes own 4 consecutive dims (one
 // u32 of int8 values), NS = 256 / (HD / 4) token slots stride the chunk,
-// and the slots are summed through LDS.
+// and the slots are summed through LDS.  The heads advance together over
+// each 4-dim piece (independent sums, one conversion of K), and a token's
+// numerators are read together; the order of every sum is that of a head by
+// itself.  Four heads of 256: 83 registers, five workgroups a CU (126 and
+// four with a head at a time over the whole converted quarter); 32000 tokens,
+// 16 heads over 2 (51 MB): 23.6 -> 23.0 us, the attention block's call 56.2
+// -> 54.5.  More in flight gave little: neither 1.8 TB/s with the partials
+// nor the vector unit's 11 us is the limit, but rounds of load, score,
+// normalise and weigh at 7.8 workgroups a CU.
 template <int G, int HD>
 __global__ void __launch_bounds__(256) k_attn_part(AttnArgs a) {
     constexpr int CH = ATTN_CHUNK;          // tokens per chunk (64)
@@ -500,7 +508,7 @@ __global__ void __launch_bounds__(256) k_attn_part(AttnArgs a) {
     constexpr int TPS = CH / NS;            // tokens per slot
     static_assert(CH * 4 == 256, "one thread quarter per token");
     __shared__ __align__(16) float sq[G][QP];
-    __shared__ float sp[G][CH];
+    __shared__ __align__(16) float sp[CH][G];  // a token's heads side by side: one read each in P.V
     __shared__ float sml[G][2];
     __shared__ __align__(16) float so[NS][G][HD];
     // x = (kv head, slice of G of its query heads): a kv head's query heads
@@ -570,49 +578,57 @@ __global__ void __launch_bounds__(256) k_attn_part(AttnArgs a) {
     __syncthreads();
 
     // ---- scores: s[g][tk] = scale * sum_blocks fp16(ks) * (q . k_int8)
-    float kf[KB][32];
-#pragma unroll
-    for (int k = 0; k < KB; ++k) {
-        const uint32_t w[8] = {kw[k][0].x, kw[k][0].y, kw[k][0].z, kw[k][0].w,
-                               kw[k][1].x, kw[k][1].y, kw[k][1].z, kw[k][1].w};
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) kf[k][j * 4 + e] = (float)(int8_t)(w[j] >> (8 * e));
-    }
+    // One q8 block of K in f32 at a time, the heads' sums side by side.
     bool vis = true;
     if (sel) {
         const uint32_t tok = t0 + tk, blk = tok / a.ratio;
         vis = blk >= nblk || ((a.vmask[(size_t)b * a.mask_words + (blk >> 5)] >> (blk & 31)) & 1u);
     }
-#pragma unroll 1
-    for (int g = 0; g < G; ++g) {
-        float v = 0.0f;
+    float sv[G];
 #pragma unroll
-        for (int k = 0; k < KB; ++k) {
-            const float4* qp = reinterpret_cast<const float4*>(&sq[g][qq * (DPT + 4) + k * 32]);
-            float acc = 0.0f;
+    for (int g = 0; g < G; ++g) sv[g] = 0.0f;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float4 qv = qp[j];
-                acc += qv.x * kf[k][4 * j] + qv.y * kf[k][4 * j + 1] + qv.z * kf[k][4 * j + 2] + qv.w * kf[k][4 * j + 3];
+    for (int k = 0; k < KB; ++k) {
+        const uint32_t w[8] = {kw[k][0].x, kw[k][0].y, kw[k][0].z, kw[k][0].w,
+                               kw[k][1].x, kw[k][1].y, kw[k][1].z, kw[k][1].w};
+        float acc[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc[g] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            float kf[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) kf[e] = (float)(int8_t)(w[j] >> (8 * e));
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const float4 qv = *reinterpret_cast<const float4*>(&sq[g][qq * (DPT + 4) + k * 32 + 4 * j]);
+                acc[g] += qv.x * kf[0] + qv.y * kf[1] + qv.z * kf[2] + qv.w * kf[3];
             }
-            v += acc * h2f(ksc[k]);
+            // (else every q read moves up front: 256 registers)
+            if (j % 2)
+#pragma unroll
+                for (int g = 0; g < G; ++g) asm volatile("" : "+v"(acc[g])::"memory");
         }
+#pragma unroll
+        for (int g = 0; g < G; ++g) sv[g] += acc[g] * h2f(ksc[k]);
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        float v = sv[g];
         v += __shfl_xor(v, 1);
         v += __shfl_xor(v, 2);
-        if (qq == 0) sp[g][tk] = tk < n && vis ? v * a.scale : -INFINITY;
+        if (qq == 0) sp[tk][g] = tk < n && vis ? v * a.scale : -INFINITY;
     }
     __syncthreads();
 
     // ---- per-head chunk softmax numerators: wave w takes heads w, w + 4, ...
     const uint32_t wv = t >> 6, lane = t & 63;
     for (uint32_t g = wv; g < (uint32_t)G; g += 4) {
-        const float s = sp[g][lane];
+        const float s = sp[lane][g];
         const float m = wave_max(s);
         // a chunk may hold no visible token (QSA): then m = -inf and p = 0
         const float p = lane < n && s != -INFINITY ? expf(s - m) : 0.0f;
-        sp[g][lane] = p;
+        sp[lane][g] = p;
         const float l = wave_sum(p);
         if (lane == 0) {
             sml[g][0] = m;
@@ -636,10 +652,15 @@ __global__ void __launch_bounds__(256) k_attn_part(AttnArgs a) {
         for (int e = 0; e < 4; ++e) vf[e] = (float)(int8_t)(vw[i] >> (8 * e)) * ds;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            const float p = sp[g][j];  // 0 past the chunk's valid tokens
+            const float p = sp[j][g];  // 0 past the chunk's valid tokens
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[g][e] += p * vf[e];
         }
+        if (i % 4 == 3)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(o[g][e])::"memory");
     }
 #pragma unroll
     for (int g = 0; g < G; ++g)
