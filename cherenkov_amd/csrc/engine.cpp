@@ -2518,33 +2518,50 @@ void ChkEngine::restore_prefix(const ChkPrefixState& cp) {
         return -1;                     \
     }
 
-// Device scratch of one primitive call, its parts on 256-byte boundaries of
-// one allocation: each hipMalloc and hipFree costs the host what a small
-// kernel takes.  8192 x 2048 over 1000 rows (83 us of kernels): 182 us a
-// call with four allocations and the codes copied, 121 with one and the
-// codes read in place; one row's head of 151936: 53 -> 52 with one for three.
+// Device scratch of one primitive call: parts on 256-byte boundaries of one
+// allocation, or of one each.  The runtime serves a request under 2 MB from
+// blocks it keeps, 1.3 us for an allocation and its release, and maps a
+// larger one anew, 13 to 24 us whatever its size.  So small parts share an
+// allocation while it stays small and get their own where the sum would not
+// (768 x 960 over 600 rows, 2.3 MB in parts of 1.1: a call 58 us with four
+// allocations, 86 with one, 56 so); a large part takes the others along
+// (8192 x 2048 over 1000 rows, two of 3.9 MB: 175 with four and the codes
+// copied, 127 so).
 struct CallScratch {
-    void* base = nullptr;
+    static constexpr size_t SMALL = 2u << 20;
+    struct Free {
+        void operator()(void* p) const { (void)hipFree(p); }
+    };
+    std::vector<std::unique_ptr<void, Free>> base;
     std::vector<void*> part;
     explicit CallScratch(std::initializer_list<size_t> bytes) {
-        size_t at = 0;
-        std::vector<size_t> start;
+        size_t sum = 0, most = 0;
         for (size_t n : bytes) {
-            start.push_back(at);
-            at += (n + 255) & ~(size_t)255;
+            sum += padded(n);
+            most = std::max(most, padded(n));
         }
-        HIPCHK(hipMalloc(&base, at));
-        for (size_t o : start) part.push_back((uint8_t*)base + o);
+        const bool shared = sum < SMALL || most >= SMALL;
+        uint8_t* at = shared ? alloc(sum) : nullptr;
+        for (size_t n : bytes) {
+            part.push_back(shared ? at : n ? alloc(n) : nullptr);
+            if (shared) at += padded(n);
+        }
     }
-    CallScratch(const CallScratch&) = delete;
-    CallScratch& operator=(const CallScratch&) = delete;
+    static size_t padded(size_t n) { return (n + 255) & ~(size_t)255; }
     void release() {
-        void* p = base;
-        base = nullptr;
-        HIPCHK(hipFree(p));
+        while (!base.empty()) {
+            void* p = base.back().release();
+            base.pop_back();
+            HIPCHK(hipFree(p));
+        }
     }
-    ~CallScratch() {
-        if (base) (void)hipFree(base);
+
+private:
+    uint8_t* alloc(size_t n) {
+        void* p = nullptr;
+        HIPCHK(hipMalloc(&p, n));
+        base.emplace_back(p);
+        return (uint8_t*)p;
     }
 };
 
@@ -3325,15 +3342,17 @@ int chk_q4_gemm(const void* w, const void* s, const void* b, uint32_t out, uint3
         const size_t wb = (size_t)out * in / 2, sb = (size_t)out * (in / 64) * 2;
         const size_t plane = (size_t)T * in * 2;
         const bool in_place = (uintptr_t)w % 16 == 0;
-        CallScratch sc({plane, plane, (size_t)T * (in / 64) * 4, sb, sb, in_place ? 0 : wb});
+        const size_t bo = CallScratch::padded(sb);
+        CallScratch sc({plane, plane, (size_t)T * (in / 64) * 4, bo + sb, in_place ? 0 : wb});
         uint4 *hi = (uint4*)sc.part[0], *lo = (uint4*)sc.part[1];
         float* xs = (float*)sc.part[2];
-        HIPCHK(hipMemcpyAsync(sc.part[3], s, sb, hipMemcpyDeviceToDevice, st));
-        HIPCHK(hipMemcpyAsync(sc.part[4], b, sb, hipMemcpyDeviceToDevice, st));
-        if (!in_place) HIPCHK(hipMemcpyAsync(sc.part[5], w, wb, hipMemcpyDeviceToDevice, st));
+        uint8_t* pack = (uint8_t*)sc.part[3];
+        HIPCHK(hipMemcpyAsync(pack, s, sb, hipMemcpyDeviceToDevice, st));
+        HIPCHK(hipMemcpyAsync(pack + bo, b, sb, hipMemcpyDeviceToDevice, st));
+        if (!in_place) HIPCHK(hipMemcpyAsync(sc.part[4], w, wb, hipMemcpyDeviceToDevice, st));
         launch_pf_xprep(x, in, T, in, hi, lo, xs, st);
-        launch_pf_gemm(Q4Mat{(const uint32_t*)(in_place ? w : sc.part[5]), (const uint16_t*)sc.part[3],
-                             (const uint16_t*)sc.part[4], out, in},
+        launch_pf_gemm(Q4Mat{(const uint32_t*)(in_place ? w : sc.part[4]), (const uint16_t*)pack,
+                             (const uint16_t*)(pack + bo), out, in},
                        hi, lo, xs, y, T, out, st);
         HIPCHK(hipStreamSynchronize(st));
         HIPCHK(hipGetLastError());
