@@ -1515,6 +1515,7 @@ struct ChkEngine {
         return std::max<uint64_t>(C * (D.topk + 1) * D.H, 2 * std::min<uint64_t>((C + 15) / 16, fa_wmax(C)) * 16 * D.nh * (2 + D.hd));
     }
     uint32_t pf_dense_rows(uint32_t T, uint32_t pos0) const;
+    bool pf_step_form(uint32_t T, uint32_t pos0) const;
     PfFlashLaunch pf_flash_launch(uint32_t T, uint32_t pos0);
     uint32_t pf_qsa_rows(uint64_t C) const;
     void pf_alloc();
@@ -2153,12 +2154,14 @@ void ChkEngine::pf_attention(const LayerDev& L, uint32_t T, uint32_t pos0, const
         // blocks the chunk completes (later chunks and decode steps read
         // them from block_k); rows past the budget have their blocks
         // scored and the top kblk selected, qsa_rows at a time, and every
-        // row attends through the flash kernel under its selection
+        // row attends through the flash kernel under its selection, or a
+        // few rows through the decode step's kernels
         set_qsa(aa, L);
         aa.iq_ready = pf.iq_ready;
         launch_attn_prep(aa, (int)T, st);
         launch_qsa_block_keys(aa, pos0 / D.ratio, (pos0 + T) / D.ratio, st);
         const uint32_t td = pf_dense_rows(T, pos0);
+        const bool steps = pf_step_form(T, pos0);
         if (td) launch_zero_f32(reinterpret_cast<float*>(pf.qsa_rows_mask), (uint64_t)td * D.mask_words, st);
         for (uint32_t r0 = td; r0 < T; r0 += pf.qsa_rows) {
             const uint32_t nr = std::min(pf.qsa_rows, T - r0);
@@ -2167,12 +2170,31 @@ void ChkEngine::pf_attention(const LayerDev& L, uint32_t T, uint32_t pos0, const
             ag.pos = pf.pos + r0;
             ag.bscore = pf.qsa_bscore;
             ag.vmask = pf.qsa_rows_mask + (uint64_t)r0 * D.mask_words;
-            launch_pf_qsa(ag, nr, (pos0 + r0 + nr) / D.ratio, st);
+            if (steps) launch_qsa(ag, (int)nr, st);
+            else launch_pf_qsa(ag, nr, (pos0 + r0 + nr) / D.ratio, st);
         }
         if (td < T) sel = PfFlashSel{pf.qsa_rows_mask, D.mask_words, D.ratio, D.kblk};
+        if (steps) {
+            // partials of as many rows as yd holds (free here, as for the
+            // flash kernel's), or of a step batch in its own buffer
+            const uint64_t fit = yd_floats(pf.cap) / ((uint64_t)D.nh * aa.max_chunks * (D.hd + 2));
+            const bool in_yd = fit >= std::min<uint32_t>(T, MAX_NB);
+            const uint32_t group = in_yd ? (uint32_t)std::min<uint64_t>(fit, T) : MAX_NB;
+            for (uint32_t r0 = 0; r0 < T; r0 += group) {
+                AttnArgs ag = aa;
+                ag.q_raw = pf.q_raw + (uint64_t)r0 * 2 * D.nh * D.hd;
+                ag.q_ready = pf.q_ready + (uint64_t)r0 * D.nh * D.hd;
+                ag.pos = pf.pos + r0;
+                ag.out = pf.attn_out + (uint64_t)r0 * D.nh * D.hd;
+                ag.vmask = pf.qsa_rows_mask + (uint64_t)r0 * D.mask_words;
+                ag.part = in_yd ? pf.yd : s.part;
+                launch_attn_core(ag, (int)std::min(group, T - r0), st);
+            }
+        }
     }
-    launch_pf_flash(pf.q_ready, pf.q_raw, kvl, pf.attn_out, T, pos0, D.nh, D.nkv, D.hd, D.attn_scale,
-                    pf_flash_launch(T, pos0), st, sel);
+    if (!pf_step_form(T, pos0))
+        launch_pf_flash(pf.q_ready, pf.q_raw, kvl, pf.attn_out, T, pos0, D.nh, D.nkv, D.hd, D.attn_scale,
+                        pf_flash_launch(T, pos0), st, sel);
     launch_pf_xprep(pf.attn_out, D.nh * D.hd, T, D.nh * D.hd, pf.hi, pf.lo, pf.xs, st);
     pf_out_proj(L.at.o, D.nh * D.hd, T);
 }
@@ -2183,6 +2205,23 @@ uint32_t ChkEngine::pf_dense_rows(uint32_t T, uint32_t pos0) const {
     if (!D.qsa) return T;
     const uint32_t first_sel = (D.kblk + 1) * D.ratio - 1;  // first position with nblk > kblk
     return first_sel <= pos0 ? 0 : std::min(T, first_sel - pos0);
+}
+
+// Whether a chunk's attention takes the decode step's kernels: few rows, all
+// past the QSA budget.  The flash kernel walks a context in 32-token steps
+// of 4.4 us over the CUs whatever the rows (up to 16) and wants its plan
+// uploaded; k_attn_part spends per row, 64 tokens and kv head a time that
+// grows with the heads (units of (g / gw) (4 + gw), gw = min(g, 4) heads a
+// workgroup).  They meet near T units = 28 + 25600 / (nkv chunks).  A whole
+// one-layer chunk behind 30000 tokens, steps / flash: 16 heads of 256 over 2,
+// 1 row 254 / 289 us, 3 rows 284 / 294, 6 rows 335 / 303; 2 over 2, 1 row
+// 226 / 271, 8 rows 284 / 284; 8 of 128 over 8, 1 row 238 / 307, 6 rows
+// 322 / 318; behind 5000, 1 row 195..220 / 215..240 in every form.
+bool ChkEngine::pf_step_form(uint32_t T, uint32_t pos0) const {
+    if (T > 16 || pf_dense_rows(T, pos0)) return false;
+    const uint32_t g = D.nh / D.nkv, gw = std::min(g, 4u);
+    const uint64_t at = (uint64_t)D.nkv * ((pos0 + T - 1) / ATTN_CHUNK + 1);
+    return (uint64_t)T * (g / gw) * (4 + gw) * at <= 28 * at + 25600;
 }
 
 // The flash plan for (T rows at pos0), made and uploaded when the key
@@ -2337,7 +2376,7 @@ void ChkEngine::prefill_gemm(const uint32_t* toks, uint32_t n, uint32_t next_aft
         // form of its sums (k_pf_flash_first)
         pf.first = pos0 == 0;
         // the chunk's flash plan, while the stream is idle
-        pf_flash_launch(T, pos0);
+        if (!pf_step_form(T, pos0)) pf_flash_launch(T, pos0);
         launch_pf_embed(pf.tokens, embed, pf.hyper, D.H, D.hc, T, st);
         for (uint32_t l = 0; l < c.num_hidden_layers; ++l) {
             const LayerDev& L = layers[l];
