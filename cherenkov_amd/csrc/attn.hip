@@ -497,8 +497,15 @@ CHK_DEV float h2f(uint16_t h) { return __half2float(__ushort_as_half(h)); }
 // -> 54.5.  More in flight gave little: neither 1.8 TB/s with the partials
 // nor the vector unit's 11 us is the limit, but rounds of load, score,
 // normalise and weigh at 7.8 workgroups a CU.
+//
+// One head of 256 dims: four workgroups a CU and free scheduling (with more
+// of them the streams slow each other).  65000 tokens, 4 heads over 4, 4
+// rows: 156 us a call with a head at a time, 172 with the accumulators pinned
+// and seven workgroups, 164 unpinned with six, 152 so.
 template <int G, int HD>
-__global__ void __launch_bounds__(256) k_attn_part(AttnArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, G == 1 && HD == 256 ? 4 : 8)))
+k_attn_part(AttnArgs a) {
+    constexpr bool PIN = G > 1 || HD < 256;  // accumulators in order (see below)
     constexpr int CH = ATTN_CHUNK;          // tokens per chunk (64)
     constexpr int DPT = HD / 4;             // score dims per thread
     constexpr int KB = DPT / 32;            // q8 blocks per thread
@@ -604,8 +611,8 @@ __global__ void __launch_bounds__(256) k_attn_part(AttnArgs a) {
                 const float4 qv = *reinterpret_cast<const float4*>(&sq[g][qq * (DPT + 4) + k * 32 + 4 * j]);
                 acc[g] += qv.x * kf[0] + qv.y * kf[1] + qv.z * kf[2] + qv.w * kf[3];
             }
-            // (else every q read moves up front: 256 registers)
-            if (j % 2)
+            // (else every q read moves up front: four heads of 256 in 256 registers)
+            if (PIN && j % 2)
 #pragma unroll
                 for (int g = 0; g < G; ++g) asm volatile("" : "+v"(acc[g])::"memory");
         }
@@ -656,7 +663,7 @@ __global__ void __launch_bounds__(256) k_attn_part(AttnArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[g][e] += p * vf[e];
         }
-        if (i % 4 == 3)
+        if (PIN && i % 4 == 3)
 #pragma unroll
             for (int g = 0; g < G; ++g)
 #pragma unroll

@@ -42,3 +42,13 @@ def test_built_library_has_no_spilling_kernel():
         if (r.get("ScratchSize", 0) or r.get("VGPRs spill", 0)) and name not in build.SCRATCH_OK:
             bad.append(line)
     assert not bad, bad
+
+
+def test_single_head_attention_partials_keep_four_waves():
+    """k_attn_part with one head of 256 dims: with seven waves a SIMD instead
+    of four, 4 rows behind 65000 tokens (4 heads over 4) took 172 us for 152."""
+    path = build.BUILD / "kernel_resources.txt"
+    if not path.exists():
+        return
+    rows = [line for line in path.read_text().splitlines() if "11k_attn_partILi1ELi256E" in line]
+    assert rows and all(ast.literal_eval(r.partition(" ")[2])["Occupancy"] == 4 for r in rows)
