@@ -220,7 +220,7 @@ struct ChkEngine {
     // low-bit form); the step graphs are recaptured when that changes
     uint32_t kinds_q4 = 0;
     uint32_t record_layers = 0;
-    uint32_t ncu = 256;  // compute units of the device (flash attention plans)
+    uint32_t ncu = 256;  // compute units of the device (prefill launch rules)
     uint64_t state_bytes = 0, kv_bytes = 0, scratch_bytes = 0;
     Q4Mat embed{}, lm_head{};
     std::vector<LayerDev> layers;
@@ -1933,7 +1933,7 @@ void ChkEngine::pf_hc_read(const HcDev& w, float* inj, uint32_t T, bool for_moe)
     g.N = N;
     g.K = D.hh;
     g.M = T;
-    g.ksplit = pf.first ? D.hc : pf_ksplit(N, D.hh, T, D.hc, (uint32_t)std::min<uint64_t>(16, std::max(act_fit, own_fit)));
+    g.ksplit = pf.first ? D.hc : pf_ksplit(N, D.hh, T, D.hc, (uint32_t)std::min<uint64_t>(16, std::max(act_fit, own_fit)), ncu);
     g.zstride = (uint64_t)T * N;
     g.xhi = pf.hi;
     g.xlo = pf.lo;
@@ -2002,7 +2002,7 @@ void ChkEngine::pf_out_proj(const Q4Mat& m, uint32_t K, uint32_t T) {
     o.N = D.H;
     o.K = K;
     o.M = T;
-    o.ksplit = G % 2 == 0 && (G / 2) % 8 == 0 ? pf_ksplit(D.H, K, T, 2, pf.first ? 2 : std::min<uint32_t>(8, D.topk + 1)) : 1;
+    o.ksplit = G % 2 == 0 && (G / 2) % 8 == 0 ? pf_ksplit(D.H, K, T, 2, pf.first ? 2 : std::min<uint32_t>(8, D.topk + 1), ncu) : 1;
     o.zstride = (uint64_t)pf.cap * D.H;
     o.xhi = pf.hi;
     o.xlo = pf.lo;
@@ -2017,7 +2017,7 @@ void ChkEngine::pf_out_proj(const Q4Mat& m, uint32_t K, uint32_t T) {
 // (in yd, free here) one pass sums into the segments.
 void ChkEngine::pf_in_proj(const PfGemmArgs& g, uint32_t T) {
     const uint64_t fit = (uint64_t)pf.cap * (D.topk + 1) * D.H / ((uint64_t)T * g.N);
-    const uint32_t ks = pf_ksplit(g.N, g.K, T, 1, (uint32_t)std::min<uint64_t>(4, fit), 2);
+    const uint32_t ks = pf_ksplit(g.N, g.K, T, 1, (uint32_t)std::min<uint64_t>(4, fit), ncu, 2);
     if (pf.first || ks < 4 || g.N % 4) {
         launch_pf_gemm_args(g, PE_STORE, (T + 63) / 64, st);
         return;
@@ -2212,7 +2212,7 @@ uint32_t ChkEngine::pf_dense_rows(uint32_t T, uint32_t pos0) const {
 // of 4.4 us over the CUs whatever the rows (up to 16) and wants its plan
 // uploaded; k_attn_part spends per row, 64 tokens and kv head a time that
 // grows with the heads (units of (g / gw) (4 + gw), gw = min(g, 4) heads a
-// workgroup).  They meet near T units = 28 + 25600 / (nkv chunks).  A whole
+// workgroup).  They meet near T units = 28 + 100 CUs / (nkv chunks).  A whole
 // one-layer chunk behind 30000 tokens, steps / flash: 16 heads of 256 over 2,
 // 1 row 254 / 289 us, 3 rows 284 / 294, 6 rows 335 / 303; 2 over 2, 1 row
 // 226 / 271, 8 rows 284 / 284; 8 of 128 over 8, 1 row 238 / 307, 6 rows
@@ -2221,7 +2221,7 @@ bool ChkEngine::pf_step_form(uint32_t T, uint32_t pos0) const {
     if (T > 16 || pf_dense_rows(T, pos0)) return false;
     const uint32_t g = D.nh / D.nkv, gw = std::min(g, 4u);
     const uint64_t at = (uint64_t)D.nkv * ((pos0 + T - 1) / ATTN_CHUNK + 1);
-    return (uint64_t)T * (g / gw) * (4 + gw) * at <= 28 * at + 25600;
+    return (uint64_t)T * (g / gw) * (4 + gw) * at <= 28 * at + 100 * ncu;
 }
 
 // The flash plan for (T rows at pos0), made and uploaded when the key
@@ -3452,6 +3452,15 @@ int chk_pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, u
 int chk_pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
                        uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge) {
     return flash_plan_out([](uint32_t t, uint32_t p, uint32_t w) { return pf_flash_split(t, p, w); }, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
+}
+
+int chk_pf_gemm_form(uint32_t N, uint32_t K, uint32_t M, uint32_t least, uint32_t most, uint32_t cus, uint32_t per_cu,
+                     uint32_t* ksplit, uint32_t* tile_rows) {
+    CHK_TRY({
+        ensure(N && K && M && least && cus && per_cu, "sizes, chunks and compute units must be positive");
+        *ksplit = pf_ksplit(N, K, M, least, most, cus, per_cu);
+        *tile_rows = pf_dense_tile_rows(N, K, M, *ksplit, cus);
+    })
 }
 
 int chk_copy_f32(float* dst, const float* src, uint64_t n, void* stream) {

@@ -501,7 +501,9 @@ void launch_pf_flash(const float* q_ready, const float* q_raw, const KvDev& kv, 
                      const PfFlashSel& sel = PfFlashSel{});
 uint32_t pf_tile_rows(const PfGemmArgs& gate_up, const PfGemmArgs& down, uint32_t T, uint32_t topk, uint32_t E);
 void launch_pf_sum_parts(const PfGemmArgs& a, const float* part, uint32_t nsplit, uint32_t T, hipStream_t st);
-uint32_t pf_ksplit(uint32_t N, uint32_t K, uint32_t T, uint32_t least, uint32_t most, uint32_t per_cu = 1);
+uint32_t pf_ksplit(uint32_t N, uint32_t K, uint32_t T, uint32_t least, uint32_t most, uint32_t cus, uint32_t per_cu = 1);
+uint32_t pf_dense_tile_rows(uint32_t N, uint32_t K, uint32_t M, uint32_t ksplit, uint32_t cus);
+uint32_t pf_cus();
 void launch_pf_gemm(const Q4Mat& w, const uint4* xhi, const uint4* xlo, const float* xs, float* y, uint32_t T,
                     uint32_t ldy, hipStream_t st);
 // [down; inject] partials -> inj and d, d staged as the up GEMM's operands

@@ -25,6 +25,7 @@
 // half operands there), the grouped experts (gpu/prefill/experts.rs:29-345),
 // the sequential scan (gpu/prefill/deltanet.rs:7-110).
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <stdexcept>
 #include <type_traits>
@@ -321,7 +322,6 @@ __global__ void __launch_bounds__(256) k_pf_hc_prep(float* __restrict__ hyper, c
 // 16 outputs: mixed = (1/hc) sum_g sigmoid(v_g) normed_g, cpu.rs:477-491),
 // PE_SILU_MUL (NMAT 2: silu(gate) * up, mlp, cpu.rs:981-992).
 constexpr int PF_WG = 256;  // threads per GEMM workgroup
-constexpr uint32_t PF_CUS = 256;  // compute units the launch rules count on
 constexpr int PF_AROW = 9;  // uint4 per staged A row (8 + 1 pad: bank spread)
 
 CHK_DEV h8 pf_unpack(uint32_t w, const Q4Consts& qk) {
@@ -1934,6 +1934,29 @@ uint32_t pf_tile_rows(const PfGemmArgs& gu, const PfGemmArgs& dn, uint32_t T, ui
     return pf_gemm_prepare(a, PE_SILU_MUL) && pf_gemm_prepare(b, PE_STORE) ? 32 : 64;
 }
 
+// Compute units of the current device, asked once per device.
+uint32_t pf_cus() {
+    static std::atomic<uint32_t> known[64];
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (const uint32_t k = known[dev].load(std::memory_order_relaxed)) return k;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
+    known[dev].store((uint32_t)n, std::memory_order_relaxed);
+    return (uint32_t)n;
+}
+
+// Rows of a dense GEMM's tiles: a launch of 64-row tiles that leaves CUs
+// without a workgroup takes 32-row tiles, twice the workgroups with little
+// over half the work each (a group's 73 unpack instructions are not shared
+// by the halves; matrix and vector instructions of a SIMD hardly overlap, so
+// a lone workgroup's step is their sum).  70 rows, 12288 outputs: 43 -> 28
+// us; 256 rows (384 workgroups on 256 CUs): 46 either way.  Chunks of at
+// most 8 groups (a [down; inject] of 16 K chunks) are short enough for three.
+uint32_t pf_dense_tile_rows(uint32_t N, uint32_t K, uint32_t M, uint32_t ksplit, uint32_t cus) {
+    const uint64_t wg = (uint64_t)((N + 255) / 256) * ((M + 31) / 32) * ksplit;
+    return wg <= cus || (K / 64 / ksplit <= 8 && wg <= 3ull * cus) ? 32 : 64;
+}
+
 bool launch_pf_gemm_args(const PfGemmArgs& args, int epi, uint32_t grid_y, hipStream_t st) {
     if (args.K % 64 || !args.K) throw std::runtime_error("prefill GEMM needs K a multiple of 64");
     if (!grid_y) return true;
@@ -1970,16 +1993,9 @@ bool launch_pf_gemm_args(const PfGemmArgs& args, int epi, uint32_t grid_y, hipSt
         if (sbl) k_pf_gemm<NM, E, true><<<dim3(GX, grid_y, ksplit), PF_WG, 0, st>>>(a); \
         else k_pf_gemm<NM, E, false><<<dim3(GX, grid_y, ksplit), PF_WG, 0, st>>>(a);    \
     } while (0)
-    // Few rows: a launch of 64-row tiles that leaves CUs without a workgroup
-    // takes 32-row tiles, twice the workgroups with little over half the
-    // work each (a group's 73 unpack instructions are not shared by the
-    // halves; matrix and vector instructions of a SIMD hardly overlap, so a
-    // lone workgroup's step is their sum).  70 rows, 12288 outputs: 43 -> 28
-    // us; 256 rows (384 workgroups): 46 either way.
     if (sbl && epi == PE_STORE && !a.tinfo) {
-        const uint32_t gx = (a.N + 255) / 256, gy = (a.M + 31) / 32;
-        if (gx * gy * ksplit <= PF_CUS || (a.K / 64 / ksplit <= 8 && gx * gy * ksplit <= 3 * PF_CUS)) {
-            k_pf_gemm<1, PE_STORE, true, 4, 2><<<dim3(gx, gy, ksplit), PF_WG, 0, st>>>(a);
+        if (pf_dense_tile_rows(a.N, a.K, a.M, ksplit, pf_cus()) == 32) {
+            k_pf_gemm<1, PE_STORE, true, 4, 2><<<dim3((a.N + 255) / 256, (a.M + 31) / 32, ksplit), PF_WG, 0, st>>>(a);
             return fused;
         }
     }
@@ -2040,10 +2056,10 @@ void launch_pf_sum_parts(const PfGemmArgs& a, const float* part, uint32_t nsplit
 // 1024 (2048 rows fill the CUs with a chunk per stream).  Out-projection
 // (4096 inputs): 43 -> 13 us at 128 rows, 21 at 256, 29 at 512.  The engine
 // asks for more than `least` behind a context only (see k_pf_flash_first).
-uint32_t pf_ksplit(uint32_t N, uint32_t K, uint32_t T, uint32_t least, uint32_t most, uint32_t per_cu) {
+uint32_t pf_ksplit(uint32_t N, uint32_t K, uint32_t T, uint32_t least, uint32_t most, uint32_t cus, uint32_t per_cu) {
     const uint32_t G = K / 64, wg = (N + 255) / 256 * ((T + 63) / 64);
     uint32_t ks = least;
-    while (2 * ks <= most && G % (2 * ks) == 0 && G / (2 * ks) % 8 == 0 && wg * 2 * ks <= per_cu * PF_CUS) ks *= 2;
+    while (2 * ks <= most && G % (2 * ks) == 0 && G / (2 * ks) % 8 == 0 && wg * 2 * ks <= per_cu * cus) ks *= 2;
     return ks;
 }
 

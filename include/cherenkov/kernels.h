@@ -226,6 +226,13 @@ int chk_pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, u
 int chk_pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
                        uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge);
 
+/* The form of a dense prefill GEMM whose consumer sums K-chunk partials
+ * (host code, no device call; a test entry point): N outputs of K inputs
+ * over M rows on `cus` compute units in `least` to `most` K chunks and at
+ * most per_cu workgroups of 64 rows a unit; *tile_rows 32 or 64. */
+int chk_pf_gemm_form(uint32_t N, uint32_t K, uint32_t M, uint32_t least, uint32_t most, uint32_t cus, uint32_t per_cu,
+                     uint32_t* ksplit, uint32_t* tile_rows);
+
 /* Time the decode step on the engine's stream: runs `steps` step_rows(1)
  * + commit pairs, returns milliseconds per step (HIP events). */
 int chk_time_decode(ChkEngine* e, uint32_t first_token, uint32_t steps, float* ms_per_step, uint32_t* last_token);
