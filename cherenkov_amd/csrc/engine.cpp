@@ -144,7 +144,7 @@ struct PfBufs {
     float* hyper;
     uint4 *hi, *lo, *bhi, *bmid, *blo;
     float* xs;
-    float *inv, *d, *inj_a, *inj_m, *mixed, *hc_part;
+    float *inv, *d, *inj_a, *inj_m, *mixed;
     uint4 *dhi, *dlo;  // d staged as the hyper-connection up GEMM's operands
     float* dxs;
     uint4 *ahi, *alo;  // the expert activations staged as the down GEMM's operands
@@ -159,7 +159,6 @@ struct PfBufs {
     // hyper-connection read: the streams it goes into, and the rows
     float* moe_pend = nullptr;
     uint32_t moe_pend_T = 0;
-    float* dcw;  // chunked-scan workspace (null: sequential scan)
     float *q_raw, *k_raw, *v_raw, *idx_raw, *q_ready, *attn_out;
     float *logits, *sg, *wts;
     uint32_t *ids, *list, *count, *tiles, *ntiles;
@@ -1499,20 +1498,43 @@ struct ChkEngine {
     uint32_t prefill_rows_fit(bool all_logits) const;
     // ------------------------------------------------- GEMM prefill
     bool pf_supported() const;
-    // flash attention plans: workgroups per kv head, segment and merge
-    // entries, partial slots (held in yd)
-    uint32_t fa_wmax(uint64_t C) const {
-        return (uint32_t)std::min<uint64_t>(8 * ((C + 15) / 16), std::max<uint32_t>(1, ncu / D.nkv));
-    }
-    uint64_t fa_entries(uint64_t C) const { return std::max<uint64_t>((C + 15) / 16, fa_wmax(C)); }
+    // The buffers of C rows hold the partials that the launch rules choose
+    // for any chunk of up to C rows: the rules see the chunk, the shape and
+    // the device only, so a chunk's sums do not depend on the capacity.
+    // Flash attention plans: workgroups per kv head, segment and merge
+    // entries, partial slots of k_pf_flash
+    uint32_t fa_wmax() const { return std::max<uint32_t>(1, ncu / D.nkv); }
     uint64_t fa_slots(uint64_t C) const {
-        const uint32_t g = D.nh / D.nkv;
-        return C * (D.topk + 1) * D.H / ((uint64_t)D.nkv * pf_flash_rows(g) * g * (2 + D.hd));
+        return pf_flash_slots((uint32_t)C, max_t, fa_wmax(), pf_flash_rows(D.nh / D.nkv));
     }
-    // yd: the expert down outputs, or a first chunk's partials of two 16-row
-    // blocks per workgroup
+    uint64_t fa_entries(uint64_t C) const { return std::max((C + 15) / 16, std::min<uint64_t>(fa_wmax(), fa_slots(C))); }
+    uint64_t fa_slot_floats() const {
+        const uint32_t g = D.nh / D.nkv;
+        return (uint64_t)D.nkv * pf_flash_rows(g) * g * (2 + D.hd);
+    }
+    // N outputs of K inputs over up to C rows: K chunks that a launch of few
+    // rows takes, as far as pf_ksplit fills the device
+    uint64_t split_floats(uint64_t C, uint64_t N, uint32_t ks, uint32_t per_cu) const {
+        return N * std::min<uint64_t>(ks * C, 64ull * per_cu * ncu / ((N + 255) / 256));
+    }
+    uint64_t hc_floats(uint64_t C) const {
+        const uint32_t N = D.lowrank + D.hc;  // (or a chunk per stream)
+        return std::max<uint64_t>(C * D.hc * N, split_floats(C, N, pf_ksplit(N, D.hh, 1, D.hc, PF_HC_SPLIT, ~0u), 1));
+    }
+    uint64_t in_floats(uint64_t C) const {
+        if (pf_ksplit(1, D.H, 1, 1, PF_IN_SPLIT, ~0u) < PF_IN_SPLIT) return 0;
+        return std::max(split_floats(C, D.conv_dim + D.v_dim, PF_IN_SPLIT, 2),
+                        split_floats(C, 2 * D.nh * D.hd + 2 * D.kv_row + D.idx_out, PF_IN_SPLIT, 2));
+    }
+    // yd: the expert down outputs; before them a layer's partials, each
+    // consumed before the next are written: the [down; inject] and the input
+    // projections', a first chunk's attention (two 16-row blocks a
+    // workgroup), k_pf_flash's; the chunked scan's workspace
     uint64_t yd_floats(uint64_t C) const {
-        return std::max<uint64_t>(C * (D.topk + 1) * D.H, 2 * std::min<uint64_t>((C + 15) / 16, fa_wmax(C)) * 16 * D.nh * (2 + D.hd));
+        return std::max<uint64_t>({C * (D.topk + 1) * D.H, hc_floats(C), in_floats(C),
+                                   2 * std::min<uint64_t>((C + 15) / 16, fa_wmax()) * 16 * D.nh * (2 + D.hd),
+                                   fa_slots(C) * fa_slot_floats(),
+                                   dc_supported(D.nk, D.nv, D.dk, D.dv) ? dc_work_floats((uint32_t)C, D.nv, D.dv) : 0});
     }
     uint32_t pf_dense_rows(uint32_t T, uint32_t pos0) const;
     bool pf_step_form(uint32_t T, uint32_t pos0) const;
@@ -1745,7 +1767,7 @@ uint64_t ChkEngine::prefill_scratch_bytes(uint64_t C, bool all_logits) const {
     if (has_mtp) b += C * 4 + C * (2ull * D.H + 3ull * D.hh) * f;
     const uint64_t plane = std::max({C * D.hh, C * D.v_dim, C * D.nh * D.hd, C * slots * D.I, C * D.SI, C * D.H});
     b += plane * 2 * 2 + plane / 64 * f + 3 * C * D.H * 2;
-    b += C * (3ull * D.hc + D.lowrank + D.H + (uint64_t)D.hc * (D.lowrank + D.hc)) * f;
+    b += C * (3ull * D.hc + D.lowrank + D.H) * f;
     b += C * D.lowrank / 8 * 32 + (C * D.lowrank / 64 + 1) * f;
     b += C * slots * D.I / 8 * 32 + (C * slots * D.I / 64 + 1) * f;
     const uint64_t dn = C * (2ull * D.conv_dim + 2ull * D.v_dim + (2ull * pf_ab_split(D.H) + 2) * D.nv);
@@ -1756,7 +1778,6 @@ uint64_t ChkEngine::prefill_scratch_bytes(uint64_t C, bool all_logits) const {
     b += (uint64_t)(pf_tile_bound((uint32_t)C, D.topk, D.E, 32)) * 12 +
          (C * slots * D.I + yd_floats(C)) * f + C * slots * 4 + (D.E + 1) * 4;
     if (D.SI != D.I) b += C * D.SI * f;
-    if (dc_supported(D.nk, D.nv, D.dk, D.dv)) b += dc_work_floats((uint32_t)C, D.nv, D.dv) * f;
     if (all_logits) b += C * D.V * f;
     b += fa_entries(C) * (FA_MAXSEG + 1) * 16;
     if (ple_l >= 0) b += C * (ngram_heads + c.ple_embed_dim + 3ull * D.hh + D.H) * 4;
@@ -1839,7 +1860,6 @@ void ChkEngine::pf_alloc() {
     pf.ahi = pfalloc<uint4>(C * slots * D.I / 8);
     pf.alo = pfalloc<uint4>(C * slots * D.I / 8);
     pf.axs = pfalloc<float>(C * slots * D.I / 64 + 1);
-    pf.hc_part = pfalloc<float>(C * D.hc * (D.lowrank + D.hc));
     pf.inj_a = pfalloc<float>(C * D.hc);
     pf.inj_m = pfalloc<float>(C * D.hc);
     pf.mixed = pfalloc<float>(C * D.H);
@@ -1884,7 +1904,6 @@ void ChkEngine::pf_alloc() {
     pf.act = pfalloc<float>(C * slots * D.I);
     pf.act_sh = D.SI != D.I ? pfalloc<float>(C * D.SI) : nullptr;
     pf.yd = pfalloc<float>(yd_floats(C));
-    pf.dcw = dc_supported(D.nk, D.nv, D.dk, D.dv) ? pfalloc<float>(dc_work_floats((uint32_t)C, D.nv, D.dv)) : nullptr;
     if (D.qsa) {
         pf.qsa_rows = pf_qsa_rows(C);
         pf.iq_ready = pfalloc<float>(C * D.inh * D.ihd);
@@ -1919,27 +1938,23 @@ void ChkEngine::pf_hc_read(const HcDev& w, float* inj, uint32_t T, bool for_moe)
                       (uint64_t)pf.cap * D.H, pf.pend_split, pf.inj_a, st, mc);
     pf.pend = nullptr;
     // [down; inject] is narrow (lowrank + hc outputs) over a long K = hc H:
-    // split K by stream, a few rows' further (as far as the partials fit),
-    // partials summed in K order by the finisher
+    // split K by stream, a few rows' further, partials (in yd, free once the
+    // pass above has read it) summed in K order by the finisher
     const uint32_t N = D.lowrank + D.hc;
-    // (the partials' buffer holds hc chunks of a full chunk's rows; the
-    // expert activations' f32 rows, free here, more at most shapes)
-    const uint64_t act_fit = (uint64_t)pf.cap * (D.topk + 1) * D.I / ((uint64_t)T * N), own_fit = (uint64_t)pf.cap * D.hc / T;
-    float* part = act_fit > own_fit ? pf.act : pf.hc_part;
     PfGemmArgs g{};
-    g.seg[0] = PfSeg{w.down, part, N, 0};
-    g.seg[1] = PfSeg{w.inject, part + D.lowrank, N, D.lowrank};
+    g.seg[0] = PfSeg{w.down, pf.yd, N, 0};
+    g.seg[1] = PfSeg{w.inject, pf.yd + D.lowrank, N, D.lowrank};
     g.nseg = 2;
     g.N = N;
     g.K = D.hh;
     g.M = T;
-    g.ksplit = pf.first ? D.hc : pf_ksplit(N, D.hh, T, D.hc, (uint32_t)std::min<uint64_t>(16, std::max(act_fit, own_fit)), ncu);
+    g.ksplit = pf.first ? D.hc : pf_ksplit(N, D.hh, T, D.hc, PF_HC_SPLIT, ncu);
     g.zstride = (uint64_t)T * N;
     g.xhi = pf.hi;
     g.xlo = pf.lo;
     g.xs = pf.xs;
     launch_pf_gemm_args(g, PE_STORE, mt, st);
-    launch_pf_hc_down_finish(part, g.ksplit, T, D.lowrank, D.hc, 1.0f / (float)D.hc, pf.d, inj, pf.dhi, pf.dlo, pf.dxs,
+    launch_pf_hc_down_finish(pf.yd, g.ksplit, T, D.lowrank, D.hc, 1.0f / (float)D.hc, pf.d, inj, pf.dhi, pf.dlo, pf.dxs,
                              st);
     PfGemmArgs u{};
     u.seg[0].m = w.up;
@@ -2016,9 +2031,8 @@ void ChkEngine::pf_out_proj(const Q4Mat& m, uint32_t K, uint32_t T) {
 // rows leave CUs idle: K then goes over up to four chunks, whose partials
 // (in yd, free here) one pass sums into the segments.
 void ChkEngine::pf_in_proj(const PfGemmArgs& g, uint32_t T) {
-    const uint64_t fit = (uint64_t)pf.cap * (D.topk + 1) * D.H / ((uint64_t)T * g.N);
-    const uint32_t ks = pf_ksplit(g.N, g.K, T, 1, (uint32_t)std::min<uint64_t>(4, fit), ncu, 2);
-    if (pf.first || ks < 4 || g.N % 4) {
+    const uint32_t ks = pf_ksplit(g.N, g.K, T, 1, PF_IN_SPLIT, ncu, 2);
+    if (pf.first || ks < PF_IN_SPLIT || g.N % 4) {
         launch_pf_gemm_args(g, PE_STORE, (T + 63) / 64, st);
         return;
     }
@@ -2087,7 +2101,9 @@ void ChkEngine::pf_deltanet(const LayerDev& L, uint32_t T) {
     a.qk_dim = D.qk_dim;
     a.v_dim = D.v_dim;
     a.qscale = D.qscale;
-    launch_pf_dn(a, pf.dcw, st);
+    // (the chunked scan's workspace is yd: the input projections' partials are
+    // summed, the out-projection's not written yet)
+    launch_pf_dn(a, dc_supported(D.nk, D.nv, D.dk, D.dv) ? pf.yd : nullptr, st);
     PfPrepArgs p{};
     p.x = pf.y;
     p.ldx = D.v_dim;
@@ -2232,8 +2248,8 @@ PfFlashLaunch ChkEngine::pf_flash_launch(uint32_t T, uint32_t pos0) {
     const uint64_t key = (uint64_t)T << 32 | pos0;
     if (key != pf.fa_key) {
         const bool first = pf.first && pf_dense_rows(T, pos0) == T;
-        const PfFlashPlan p = first ? pf_flash_plan(T, 0, std::max<uint32_t>(1, ncu / D.nkv))
-                                    : pf_flash_split(T, pos0, fa_wmax(pf.cap), pf_flash_rows(D.nh / D.nkv), fa_slots(pf.cap));
+        const PfFlashPlan p = first ? pf_flash_plan(T, 0, fa_wmax())
+                                    : pf_flash_split(T, pos0, fa_wmax(), pf_flash_rows(D.nh / D.nkv));
         const uint64_t n = fa_entries(pf.cap);
         const uint64_t slots = first ? yd_floats(pf.cap) / (16ull * D.nh * (2 + D.hd)) : fa_slots(pf.cap);
         if (p.seg.size() > n * FA_MAXSEG || p.merge.size() > n || p.nslots > slots)

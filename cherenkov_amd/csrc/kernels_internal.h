@@ -478,11 +478,14 @@ struct PfFlashPlan {
 // rows of a row block: a workgroup's eight waves serve `g` query heads
 constexpr uint32_t pf_flash_rows(uint32_t g) { return g >= 8 ? 16u : 16u * (8u / g); }
 // (a prompt's first chunk, see pf_flash_first, takes this plan over 16-row blocks)
-PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows = 16, bool whole_only = false);
+PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows = 16);
 // the plan behind a context or past the QSA budget: pf_flash_plan, or where
 // the chunk has fewer row blocks than max_wg, its steps over more workgroups
-// than row blocks; at most max_slots partial slots
-PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows = 16, uint64_t max_slots = ~0ull);
+// than row blocks
+PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows = 16);
+// partial slots that pf_flash_split's plan of any chunk of up to T rows takes
+// within `ctx` tokens
+uint32_t pf_flash_slots(uint32_t T, uint32_t ctx, uint32_t max_wg, uint32_t rows);
 struct PfFlashLaunch {         // a plan uploaded to the device
     const uint4* seg;
     const uint4* merge;
@@ -501,6 +504,8 @@ void launch_pf_flash(const float* q_ready, const float* q_raw, const KvDev& kv, 
                      const PfFlashSel& sel = PfFlashSel{});
 uint32_t pf_tile_rows(const PfGemmArgs& gate_up, const PfGemmArgs& down, uint32_t T, uint32_t topk, uint32_t E);
 void launch_pf_sum_parts(const PfGemmArgs& a, const float* part, uint32_t nsplit, uint32_t T, hipStream_t st);
+// K chunks at most of the [down; inject] and the input projections' GEMMs
+constexpr uint32_t PF_HC_SPLIT = 16, PF_IN_SPLIT = 4;
 uint32_t pf_ksplit(uint32_t N, uint32_t K, uint32_t T, uint32_t least, uint32_t most, uint32_t cus, uint32_t per_cu = 1);
 uint32_t pf_dense_tile_rows(uint32_t N, uint32_t K, uint32_t M, uint32_t ksplit, uint32_t cus);
 uint32_t pf_cus();

@@ -2959,7 +2959,7 @@ __global__ void __launch_bounds__(256) k_pf_first_merge(PfFlashArgs a, const uin
 // equal shares (see k_pf_flash); one whole row block per workgroup, heavy
 // ones first, where the blocks' work is within 15% of even or a share
 // would need more than FA_MAXSEG segments.
-PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows, bool whole_only) {
+PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows) {
     PfFlashPlan p;
     const uint32_t R = (T + rows - 1) / rows;
     std::vector<uint32_t> tiles(R);
@@ -2981,7 +2981,7 @@ PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t r
         }
         return p;
     };
-    if (whole_only || (double)most <= 1.15 * (double)total / W) return whole();
+    if ((double)most <= 1.15 * (double)total / W) return whole();
     p.W = W;
     p.seg.assign((size_t)W * FA_MAXSEG, make_uint4(~0u, 0, 0, 0));
     std::vector<uint32_t> order;
@@ -3026,19 +3026,14 @@ PfFlashPlan pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t r
 // workgroups: 673 us a layer, against 48 split + 8 to join; 333 behind 1500:
 // 264 -> 67 + 12.
 // A range costs its queries and its partial once, about two tiles' time.
-PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows, uint64_t max_slots) {
+PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows) {
     const uint32_t R = (T + rows - 1) / rows;
     std::vector<uint64_t> first(R + 1, 0);
     for (uint32_t rb = 0; rb < R; ++rb)
         first[rb + 1] = first[rb] + (pos0 + std::min(rb * rows + rows - 1, T - 1)) / FA_TOK + 1;
     const uint64_t total = first[R];
-    const uint32_t W = (uint32_t)std::min<uint64_t>(
-        {max_wg, total / FA_MINSHARE, (uint64_t)FA_MAXJOIN - 1, max_slots > R ? max_slots - R : 0});
-    auto even = [&]() {
-        PfFlashPlan p = pf_flash_plan(T, pos0, max_wg, rows);
-        return p.nslots <= max_slots ? p : pf_flash_plan(T, pos0, R, rows, true);
-    };
-    if (R >= max_wg || W <= R) return even();
+    const uint32_t W = (uint32_t)std::min<uint64_t>({max_wg, total / FA_MINSHARE, (uint64_t)FA_MAXJOIN - 1});
+    if (R >= max_wg || W <= R) return pf_flash_plan(T, pos0, max_wg, rows);
     PfFlashPlan p;
     p.W = W;
     p.seg.assign((size_t)W * FA_MAXSEG, make_uint4(~0u, 0, 0, 0));
@@ -3053,13 +3048,29 @@ PfFlashPlan pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t 
         for (; k < W && k * total / W < first[rb + 1]; ++k) {
             const uint64_t lo = std::max(first[rb], k * total / W), hi = std::min(first[rb + 1], (k + 1) * total / W);
             if (lo >= hi) continue;
-            if (nseg[k] == FA_MAXSEG) return even();
+            if (nseg[k] == FA_MAXSEG) return pf_flash_plan(T, pos0, max_wg, rows);
             p.seg[(size_t)k * FA_MAXSEG + nseg[k]++] =
                 make_uint4(rb, (uint32_t)(lo - first[rb]), (uint32_t)(hi - first[rb]), split ? p.nslots++ : ~0u);
         }
         if (split) p.merge.push_back(make_uint4(rb, slot0, p.nslots - slot0, 0));
     }
     return p;
+}
+
+// W ranges make W - 1 cuts, and a block with c of them c + 1 pieces: fewer
+// than W + R over R blocks, at most 2 (W - 1).  A chunk of R blocks has at
+// most the steps it has as the context's last one.
+uint32_t pf_flash_slots(uint32_t T, uint32_t ctx, uint32_t max_wg, uint32_t rows) {
+    uint64_t most = 0, total = 0;
+    for (uint32_t R = 1; R <= (T + rows - 1) / rows; ++R) {
+        // (the last block ends with the context and may hold one row, each
+        // earlier one ends `rows` before the next)
+        const uint32_t back = R == 1 ? 0 : 1 + (R - 2) * rows;
+        total += ctx > back ? (ctx - back - 1) / FA_TOK + 1 : 1;
+        const uint64_t W = std::min<uint64_t>({max_wg, total / FA_MINSHARE, FA_MAXJOIN - 1});
+        most = std::max<uint64_t>(most, R < max_wg && W > R ? W - 1 + R : 2 * (std::min(R, max_wg) - 1));
+    }
+    return (uint32_t)most;
 }
 
 void launch_pf_flash(const float* q_ready, const float* q_raw, const KvDev& kv, float* out, uint32_t T, uint32_t pos0,

@@ -46,12 +46,12 @@ def test_few_rows_past_the_budget(have_gpu, nh, nkv, hd, budget, ratio, ctx, row
     check_chunks(config(nh, nkv, hd, budget, ratio), ctx, rows)
 
 
-# yd of 4096 rows of two outputs of 256 (2 M floats): partials of 16 heads of
-# 128 for five rows behind 12000 tokens (seven rows: two launches), for three
-# behind 16400 (then a step batch's buffer, four rows a launch)
-@pytest.mark.parametrize("ctx,rows", [(12000, (5, 7)), (16400, (1, 4, 6))])
+# 64 heads of 128 over 64: the expert output buffer holds partials of five
+# rows behind 12000 tokens (six rows: two launches), of three behind 16400
+# (then a step batch's buffer, four rows a launch)
+@pytest.mark.parametrize("ctx,rows", [(12000, (5, 6)), (16400, (1, 4, 5))])
 def test_step_form_partials_in_each_buffer(have_gpu, ctx, rows):
-    cfg = config(16, 16, 128, 63, 3)
+    cfg = config(64, 64, 128, 63, 3)
     cfg.hidden_size, cfg.num_experts_per_tok = 256, 1
     check_chunks(cfg, ctx, rows)
 
