@@ -205,6 +205,8 @@ SIGNATURES = [
     ("chk_prefix_read", i32, [P, u32, P, u64]),
     ("chk_fill_u8", i32, [P, u32, u64, P]),
     ("chk_copy_f32", i32, [P, P, u64, P]),
+    ("chk_pf_flash_split_rows", i32, [u32, u32, u32, u32, C.POINTER(u32), C.POINTER(u32), P, u64, P, u64, C.POINTER(u32)]),
+    ("chk_pf_flash_slots", i32, [u32, u32, u32, u32, C.POINTER(u32)]),
     ("chk_pf_gemm_form", i32, [u32, u32, u32, u32, u32, u32, u32, C.POINTER(u32), C.POINTER(u32)]),
     ("chk_pf_flash_plan", i32, [u32, u32, u32, C.POINTER(u32), C.POINTER(u32), P, u64, P, u64, C.POINTER(u32)]),
     ("chk_pf_flash_split", i32, [u32, u32, u32, C.POINTER(u32), C.POINTER(u32), P, u64, P, u64, C.POINTER(u32)]),

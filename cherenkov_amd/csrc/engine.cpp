@@ -3445,29 +3445,41 @@ int chk_fill_u8(void* dst, uint32_t value, uint64_t n, void* stream) {
     })
 }
 
-static int flash_plan_out(PfFlashPlan (*make)(uint32_t, uint32_t, uint32_t), uint32_t T, uint32_t pos0, uint32_t max_wg,
-                          uint32_t* W, uint32_t* nslots, uint32_t* seg, uint64_t seg_cap, uint32_t* merge,
-                          uint64_t merge_cap, uint32_t* nmerge) {
+static int flash_plan_out(PfFlashPlan (*make)(uint32_t, uint32_t, uint32_t, uint32_t), uint32_t rows, uint32_t T,
+                          uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg, uint64_t seg_cap,
+                          uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge) {
     CHK_TRY({
-        ensure(T >= 1 && max_wg >= 1, "T and max_wg must be positive");
-        const PfFlashPlan p = make(T, pos0, max_wg);
+        ensure(T >= 1 && max_wg >= 1 && rows >= 1, "T, max_wg and rows must be positive");
+        const PfFlashPlan p = make(T, pos0, max_wg, rows);
         ensure(p.seg.size() * 4 <= seg_cap && p.merge.size() * 4 <= merge_cap, "plan buffers too small");
         *W = p.W;
         *nslots = p.nslots;
         *nmerge = (uint32_t)p.merge.size();
         memcpy(seg, p.seg.data(), p.seg.size() * sizeof(uint4));
-        if (!p.merge.empty()) memcpy(merge, p.merge.data(), p.merge.size() * sizeof(uint4));
+        memcpy(merge, p.merge.data(), p.merge.size() * sizeof(uint4));
     })
 }
 
 int chk_pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
                       uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge) {
-    return flash_plan_out([](uint32_t t, uint32_t p, uint32_t w) { return pf_flash_plan(t, p, w); }, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
+    return flash_plan_out(pf_flash_plan, 16, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
 }
 
 int chk_pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
                        uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge) {
-    return flash_plan_out([](uint32_t t, uint32_t p, uint32_t w) { return pf_flash_split(t, p, w); }, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
+    return flash_plan_out(pf_flash_split, 16, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
+}
+
+int chk_pf_flash_split_rows(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows, uint32_t* W, uint32_t* nslots,
+                            uint32_t* seg, uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge) {
+    return flash_plan_out(pf_flash_split, rows, T, pos0, max_wg, W, nslots, seg, seg_cap, merge, merge_cap, nmerge);
+}
+
+int chk_pf_flash_slots(uint32_t T, uint32_t ctx, uint32_t max_wg, uint32_t rows, uint32_t* slots) {
+    CHK_TRY({
+        ensure(T >= 1 && max_wg >= 1 && rows >= 1, "T, max_wg and rows must be positive");
+        *slots = pf_flash_slots(T, ctx, max_wg, rows);
+    })
 }
 
 int chk_pf_gemm_form(uint32_t N, uint32_t K, uint32_t M, uint32_t least, uint32_t most, uint32_t cus, uint32_t per_cu,

@@ -550,10 +550,10 @@ void launch_attn_prep(const AttnArgs& a, int nb, hipStream_t st);
 void launch_qsa_select(const AttnArgs& a, int nb, hipStream_t st);
 // block keys + scores + selection of nb rows (a no-op without QSA)
 void launch_qsa(const AttnArgs& a, int nb, hipStream_t st);
-// pooled keys of blocks [blk0, blk1) of kv[0]'s sequence
 // scores and selection of nr prefill rows (a.pos their positions, block keys
 // cached, at most nblk complete blocks) into a.bscore and a.vmask
 void launch_pf_qsa(const AttnArgs& a, uint32_t nr, uint32_t nblk, hipStream_t st);
+// pooled keys of blocks [blk0, blk1) of kv[0]'s sequence
 void launch_qsa_block_keys(const AttnArgs& a, uint32_t blk0, uint32_t blk1, hipStream_t st);
 void launch_attn_core(const AttnArgs& a, int nb, hipStream_t st);
 bool attn_shape_ok(uint32_t nh, uint32_t nkv, uint32_t hd);

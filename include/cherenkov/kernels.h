@@ -219,12 +219,20 @@ int chk_time_blocks(ChkEngine* e, int kind, uint32_t nb, const uint32_t* layers,
  * partial slots. */
 int chk_pf_flash_plan(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
                       uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge);
-/* The plan the engine launches, in the same form: chk_pf_flash_plan's, or
- * where the chunk has fewer 16-row blocks than max_wg, its steps cut over
- * up to max_wg workgroups, a row block over any number of them (W <=
- * max_wg, slots < W + row blocks). */
+/* The plan of a chunk behind a context or past the QSA budget, in the same
+ * form, over 16-row blocks (a first chunk within the budget takes
+ * chk_pf_flash_plan's): chk_pf_flash_plan's, or where the chunk has fewer
+ * row blocks than max_wg, its steps cut over up to max_wg workgroups, a row
+ * block over any number of them (W <= max_wg, slots < W + row blocks). */
 int chk_pf_flash_split(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t* W, uint32_t* nslots, uint32_t* seg,
                        uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge);
+/* The same over row blocks of `rows` rows, as the engine cuts them (16 for 8
+ * query heads a kv head, 32, 64 and 128 for 4, 2 and 1). */
+int chk_pf_flash_split_rows(uint32_t T, uint32_t pos0, uint32_t max_wg, uint32_t rows, uint32_t* W, uint32_t* nslots,
+                            uint32_t* seg, uint64_t seg_cap, uint32_t* merge, uint64_t merge_cap, uint32_t* nmerge);
+/* Partial slots the engine keeps for those plans: no chunk of up to T rows
+ * that ends within `ctx` tokens takes more. */
+int chk_pf_flash_slots(uint32_t T, uint32_t ctx, uint32_t max_wg, uint32_t rows, uint32_t* slots);
 
 /* The form of a dense prefill GEMM whose consumer sums K-chunk partials
  * (host code, no device call; a test entry point): N outputs of K inputs

@@ -1,7 +1,9 @@
 """Prefill attention behind contexts of thousands of tokens, on one layer of
-a small model: chunks of a few rows past the QSA budget in the decode step's
-kernels and in the flash kernel, at the rule's line and with partials in
-each of their buffers.  Chunk and row path start from the same checkpoint."""
+a small model: row blocks joined from dozens of pieces, block scores of more
+than one workgroup and row group, and chunks of a few rows past the QSA
+budget in the decode step's kernels and in the flash kernel, at the rule's
+line and with partials in each of their buffers.  Chunk and row path start
+from the same checkpoint."""
 
 from __future__ import annotations
 
@@ -12,6 +14,7 @@ import pytest
 
 from cherenkov_amd.engine import Engine
 from tests.gpu_util import assert_close, torch_dev
+from tests.test_flash_split_rows import split
 from tests.test_gpu_flash import config
 
 pytestmark = pytest.mark.gpu
@@ -36,6 +39,23 @@ def check_chunks(cfg, ctx, rows):
                 assert_close(e.pf_logits_row(r), ref[r], f"{n} rows behind {ctx}: row {r}", abs_frac=1e-3, min_cos=0.99999)
     finally:
         e.close()
+
+
+# k_pf_flash_join: more pieces than the four it loads at once, and than the 64
+# lanes of a wave hold
+@pytest.mark.parametrize("nh,nkv,hd", [(16, 2, 256), (8, 2, 128), (4, 2, 256), (2, 2, 128)])
+@pytest.mark.parametrize("ctx,rows,more_than", [(700, (1, 16, 17, 40), 4), (6500, (1, 16, 17), 64)])
+def test_blocks_of_many_pieces(have_gpu, nh, nkv, hd, ctx, rows, more_than):
+    block = 16 * (8 // (nh // nkv))
+    _, _, _, merge = split(min(rows[-1], block), ctx, 256 // nkv, block)
+    assert merge[0][2] > more_than
+    check_chunks(config(nh, nkv, hd), ctx, rows)
+
+
+# the scores of rows past the budget stand in a buffer of 64 rows' attention
+# partials: 9 MB here, 325 rows of 6908 blocks, so 400 rows take two groups
+def test_scores_of_two_row_groups(have_gpu):
+    check_chunks(config(2, 2, 128, 64, 1), 6500, (400,))
 
 
 # the step form holds up to 16 rows behind 700 tokens, 9 (16 heads over 2)
