@@ -2598,7 +2598,7 @@ struct CallScratch {
         const bool shared = sum < SMALL || most >= SMALL;
         uint8_t* at = shared ? alloc(sum) : nullptr;
         for (size_t n : bytes) {
-            part.push_back(shared ? at : n ? alloc(n) : nullptr);
+            part.push_back(shared ? at : alloc(n));
             if (shared) at += padded(n);
         }
     }
@@ -3397,16 +3397,16 @@ int chk_q4_gemm(const void* w, const void* s, const void* b, uint32_t out, uint3
         const size_t wb = (size_t)out * in / 2, sb = (size_t)out * (in / 64) * 2;
         const size_t plane = (size_t)T * in * 2;
         const bool in_place = (uintptr_t)w % 16 == 0;
-        const size_t bo = CallScratch::padded(sb);
-        CallScratch sc({plane, plane, (size_t)T * (in / 64) * 4, bo + sb, in_place ? 0 : wb});
+        const size_t so = in_place ? 0 : CallScratch::padded(wb), bo = so + CallScratch::padded(sb);
+        CallScratch sc({plane, plane, (size_t)T * (in / 64) * 4, bo + sb});
         uint4 *hi = (uint4*)sc.part[0], *lo = (uint4*)sc.part[1];
         float* xs = (float*)sc.part[2];
         uint8_t* pack = (uint8_t*)sc.part[3];
-        HIPCHK(hipMemcpyAsync(pack, s, sb, hipMemcpyDeviceToDevice, st));
+        HIPCHK(hipMemcpyAsync(pack + so, s, sb, hipMemcpyDeviceToDevice, st));
         HIPCHK(hipMemcpyAsync(pack + bo, b, sb, hipMemcpyDeviceToDevice, st));
-        if (!in_place) HIPCHK(hipMemcpyAsync(sc.part[4], w, wb, hipMemcpyDeviceToDevice, st));
+        if (!in_place) HIPCHK(hipMemcpyAsync(pack, w, wb, hipMemcpyDeviceToDevice, st));
         launch_pf_xprep(x, in, T, in, hi, lo, xs, st);
-        launch_pf_gemm(Q4Mat{(const uint32_t*)(in_place ? w : sc.part[4]), (const uint16_t*)pack,
+        launch_pf_gemm(Q4Mat{(const uint32_t*)(in_place ? w : pack), (const uint16_t*)(pack + so),
                              (const uint16_t*)(pack + bo), out, in},
                        hi, lo, xs, y, T, out, st);
         HIPCHK(hipStreamSynchronize(st));

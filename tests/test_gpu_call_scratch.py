@@ -38,7 +38,7 @@ def test_gemm_is_one_result_for_any_split_of_its_scratch(have_gpu, rows):
     (_, _, _, _, y), x, (w, s, b), call = make(rows)
     call()
     got = to_host(y)
-    (_, _, _, _, y1), _, _, call1 = make(rows, shift=1)  # codes copied: one part more
+    (_, _, _, _, y1), _, _, call1 = make(rows, shift=1)  # codes copied: a larger part
     call1()
     assert np.array_equal(got, to_host(y1))
     sc = np.repeat((s.astype(np.uint32) << 16).view(np.float32), 64, 1).astype(np.float64)
