@@ -2121,8 +2121,8 @@ void ChkEngine::pf_deltanet(const LayerDev& L, uint32_t T) {
 
 // attention (cpu.rs:544-641) over the chunk: projections as one GEMM, the
 // per-row prep writing the chunk's q8 K/V and index keys at their
-// positions, causal attention of every row over the cache (sub-batches of
-// rows sized to the partials buffer), o-projection + inject.
+// positions, causal attention of every row over the cache, o-projection +
+// inject.
 void ChkEngine::pf_attention(const LayerDev& L, uint32_t T, uint32_t pos0, const KvDev* kvo) {
     const KvDev& kvl = kvo ? *kvo : kv[L.at_idx];
     const uint32_t mt = (T + 63) / 64;

@@ -2670,9 +2670,10 @@ __global__ void __launch_bounds__(256) k_pf_flash_join(PfFlashArgs a, const uint
 // 2048 rows of 16 heads of 256 over 2: 180 + 19 us (k_pf_flash 156 + 14,
 // 0.3 ms of a 48-layer prompt's 65).  It stays for its sums: a prompt's
 // roundings choose the cache codes and near-tied experts that its answer
-// goes on with, so a prompt answers as before (48 layers behind 2048
-// tokens: logits 3.5e-3 apart between the two forms, each within 1.8e-6 of
-// 64 bits over one layer).
+// goes on with (48 layers behind 2048 tokens: logits 3.5e-3 apart between
+// the two forms, each within 1.8e-6 of 64 bits over one layer).  A prompt of
+// one chunk within the budget keeps the sums it had; from a second chunk on
+// a prompt takes k_pf_flash like any message behind a context.
 template <int HD, int G>
 __global__ void __launch_bounds__(64 * G) k_pf_flash_first(PfFlashArgs a) {
     constexpr int KS = HD / 32;          // dim steps of 32
